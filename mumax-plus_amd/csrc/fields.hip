@@ -442,6 +442,16 @@ __global__ void __launch_bounds__(BLOCK) k_field(FMDesc d, const float* __restri
   field_body<UNI>(d, m, hdemag, out, mode, xcd_remap(blockIdx.x, gridDim.x));
 }
 
+// k_field that also writes the next Runge-Kutta stage state (nx, NK
+// derivatives from memory: a compile-time count keeps their loads in flight
+// together).
+template <bool UNI, int NK>
+__global__ void __launch_bounds__(BLOCK) k_field_next(FMDesc d, const float* __restrict__ m,
+                                                      const float* __restrict__ hdemag, float* __restrict__ out,
+                                                      NextStage nx, int mode) {
+  field_body<UNI, NK>(d, m, hdemag, out, mode, xcd_remap(blockIdx.x, gridDim.x), &nx);
+}
+
 // Both sublattices of an antiferromagnet in one launch: blockIdx.y selects
 // one.  Each branch reads its own kernel argument at fixed offsets (indexing
 // a descriptor array by blockIdx.y would copy it to scratch).
@@ -507,7 +517,9 @@ __global__ void __launch_bounds__(BLOCK) k_torque_pair(FMDesc d0, const float* _
   else torque_cell(d1, m1, hl1, hd1, o1, mode, idx);
 }
 
-template <bool NEXT>
+// NK >= 0: also the next stage state, from NK derivatives in memory and the
+// one just computed; NK == -2: none.
+template <int NK>
 __global__ void __launch_bounds__(BLOCK) k_field_uniform(FMDesc d, FMUniform u, const float* __restrict__ m,
                                                          const float* __restrict__ hdemag, float* __restrict__ out,
                                                          int mode, NextStage next) {
@@ -529,7 +541,10 @@ __global__ void __launch_bounds__(BLOCK) k_field_uniform(FMDesc d, FMUniform u, 
     const int z = (rest / nby) * MPA_FIELD_ZPER + k;
     if (z < d.nz) {
       auto hd = [&](int i) { return load3(hdemag, i, N); };
-      if constexpr (NEXT) field_uniform_cell(d, u, m, hd, out, mode, x, y, z, N, next);
+      if constexpr (NK >= 0)
+        field_uniform_cell(d, u, m, hd, out, mode, x, y, z, N, [&](int idx, float3 mc, float3 r, bool in) {
+          next.template apply<NK>(idx, mc, r, in);
+        });
       else field_uniform_cell(d, u, m, hd, out, mode, x, y, z, N);
     }
   }
@@ -1030,13 +1045,18 @@ void launch_field_uniform(const FMDesc& d, const float* m, const float* hdemag, 
   while (bx < d.nx && bx < MPA_FIELD_TILE_X) bx <<= 1;
   const int by = BLOCK / bx;
   dim3 grid((d.nx + bx - 1) / bx, (d.ny + by - 1) / by, (d.nz + MPA_FIELD_ZPER - 1) / MPA_FIELD_ZPER);
-  if (next) {
-    k_field_uniform<true><<<grid, dim3(bx, by, 1), 0, s>>>(d, u, m, hdemag, out, (int)mode, *next);
-    checkLaunch("k_field_uniform<next>");
-  } else {
-    k_field_uniform<false><<<grid, dim3(bx, by, 1), 0, s>>>(d, u, m, hdemag, out, (int)mode, NextStage{});
-    checkLaunch("k_field_uniform");
+  const dim3 blk(bx, by, 1);
+  const NextStage ns = next ? *next : NextStage{};
+  switch (next ? ns.nk : -2) {
+    case 0: k_field_uniform<0><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); break;
+    case 1: k_field_uniform<1><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); break;
+    case 2: k_field_uniform<2><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); break;
+    case 3: k_field_uniform<3><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); break;
+    case 4: k_field_uniform<4><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); break;
+    case 5: k_field_uniform<5><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); break;
+    default: k_field_uniform<-2><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); break;
   }
+  checkLaunch("k_field_uniform");
 }
 }  // namespace
 
@@ -1062,15 +1082,33 @@ void field_tile_clear() {
 }
 
 bool field_next_fusable(const FMDesc& d, FieldMode mode) {
-  return mode == MODE_LLG && all_uniform(d) && d.nz <= 65535;
+  return mode == MODE_LLG && !d.sublattice && !d.noise && (!all_uniform(d) || d.nz <= 65535);
 }
 
 void launch_field_next(const FMDesc& d, const float* m, const float* hdemag, float* out, FieldMode mode,
                        const NextStage& next, hipStream_t s) {
-  if (!field_next_fusable(d, mode)) throw Error(MPA_ERR_RUNTIME, "launch_field_next: not the uniform LLG path");
-  if (next.nk < 0 || next.nk > 7 || !next.out || next.out == m || next.out == out || next.out == next.x0)
+  if (!field_next_fusable(d, mode)) throw Error(MPA_ERR_RUNTIME, "launch_field_next: not a fusable magnet");
+  if (next.nk < 0 || next.nk > 5 || !next.out || next.out == m || next.out == out || next.out == next.x0)
     throw Error(MPA_ERR_RUNTIME, "launch_field_next: bad stage combination");
-  launch_field_uniform(d, m, hdemag, out, mode, &next, s);
+  if (all_uniform(d)) {
+    launch_field_uniform(d, m, hdemag, out, mode, &next, s);
+    return;
+  }
+  const int nblk = (d.ncell + BLOCK - 1) / BLOCK;
+  const bool u = params_uniform(d);
+#define MPA_FIELD_NEXT(K)                                                                       \
+  if (u) k_field_next<true, K><<<nblk, BLOCK, 0, s>>>(d, m, hdemag, out, next, (int)mode);      \
+  else k_field_next<false, K><<<nblk, BLOCK, 0, s>>>(d, m, hdemag, out, next, (int)mode);
+  switch (next.nk) {
+    case 0: MPA_FIELD_NEXT(0) break;
+    case 1: MPA_FIELD_NEXT(1) break;
+    case 2: MPA_FIELD_NEXT(2) break;
+    case 3: MPA_FIELD_NEXT(3) break;
+    case 4: MPA_FIELD_NEXT(4) break;
+    default: MPA_FIELD_NEXT(5) break;
+  }
+#undef MPA_FIELD_NEXT
+  checkLaunch("k_field_next");
 }
 
 void launch_field(const FMDesc& d, const float* m, const float* hdemag, float* out, FieldMode mode, hipStream_t s) {

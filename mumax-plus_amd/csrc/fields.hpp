@@ -109,9 +109,6 @@ struct NextStage {
   int nk;
   float* out;
   int N;
-  __device__ __forceinline__ void operator()(int idx, float3 mc, float3 r, bool in) const {
-    apply<-1>(idx, mc, r, in);
-  }
   // NK >= 0: nk == NK known at compile time, so every load is issued before
   // the sums (NK < 0: nk read at run time).
   template <int NK>
@@ -135,9 +132,10 @@ struct NextStage {
   }
 };
 
-// launch_field on the uniform-parameter LLG path that also writes the next
-// Runge-Kutta stage state (NextStage above); field_next_fusable
-// tells whether a magnet is on that path.
+// launch_field of a magnet's LLG torque that also writes the next
+// Runge-Kutta stage state (NextStage above, 0 to 5 derivatives from memory):
+// any ferromagnet that is no sublattice and adds no thermal noise
+// (field_next_fusable).
 bool field_next_fusable(const FMDesc& d, FieldMode mode);
 void launch_field_next(const FMDesc& d, const float* m, const float* hdemag, float* out, FieldMode mode,
                        const NextStage& next, hipStream_t s);

@@ -1775,13 +1775,14 @@ void TimeSolver::step() {
       noisy = true;
     }
   bool k0_valid = !noisy && fsal_valid_ && fsal_version_ == world_->version && fsal_time_ == t0;
-  // One independent magnet on the uniform-parameter LLG path with a
-  // first-same-as-last tableau: each evaluation also writes the next stage
-  // state (the combination's last derivative is the one just computed), so
-  // no separate combination launch runs.  With a fixed step the step's last
-  // evaluation writes the next step's first stage state as well.
+  // One independent magnet without thermal noise: each evaluation also writes
+  // the next stage state (the combination's last derivative is the one just
+  // computed), so no separate combination launch runs.  The step's last
+  // evaluation writes the next step's first stage state (first-same-as-last
+  // tableaus with a fixed step) or the step's final state (the other
+  // tableaus).
   Ferromagnet* fused = nullptr;
-  if (fuse_stages && !noisy && tb.fsal && S > 1 && vars.size() == 1 && vars[0].kind == StateVar::MAG && !world_->relaxing() &&
+  if (fuse_stages && !noisy && S > 1 && vars.size() == 1 && vars[0].kind == StateVar::MAG && !world_->relaxing() &&
       vars[0].fm->next_fusable())
     fused = vars[0].fm;
   // One independent magnetisation with demag: each stage state is formed in
@@ -1823,13 +1824,16 @@ void TimeSolver::step() {
   // x0 = the state at the step start.  When the first stage's derivative is
   // reused, nothing reads the state before the second stage's combination
   // overwrites it, so the state array and x0 trade buffers instead of copying.
+  // A fused first evaluation reads the state as its own x0, and the buffers
+  // are traded after it.
+  bool trade_x0 = fused && !k0_valid;
   for (auto& sv : vars) {
     if (sv.x0->n == 0) sv.x0->allocate((size_t)3 * sv.N);
     while ((int)sv.k->size() < S) sv.k->emplace_back((size_t)3 * sv.N);
     if (k0_valid && S > 1) {
       std::swap(*sv.xa, *sv.x0);
       sv.x = sv.xa->get();
-    } else {
+    } else if (!trade_x0) {
       Timed t(prof, "copy_x0", 24.0 * sv.N, s);
       HIP_CHECK(hipMemcpyAsync(sv.x0->get(), sv.x, (size_t)3 * sv.N * sizeof(float), hipMemcpyDeviceToDevice, s));
     }
@@ -1909,23 +1913,33 @@ void TimeSolver::step() {
         }
       }
       if (st == 0 && k0_valid) continue;
-      const bool cross = st + 1 == S;  // the next step's first stage
+      const bool last = st + 1 == S;
+      const bool cross = last && tb.fsal;  // the next step's first stage
       if (fused && !(cross && adaptive)) {
         NextStage ns{};
-        const std::vector<double>& a = tb.A[cross ? 1 : st + 1];
-        ns.x0 = cross ? nullptr : vars[0].x0->get();
-        ns.nk = cross ? 0 : st;
-        for (int j = 0; j < ns.nk; ++j) {
-          ns.k[j] = (*vars[0].k)[j].get();
-          ns.c[j] = (float)(h * a[j]);
-        }
+        const std::vector<double>& a = cross ? tb.A[1] : (last ? tb.w1 : tb.A[st + 1]);
+        const bool own = cross || trade_x0;  // the evaluated state is the combination's x0
+        ns.x0 = own ? nullptr : vars[0].x0->get();
+        if (!cross)
+          for (int j = 0; j < st; ++j) {
+            if (a[j] == 0.0) continue;  // adds an exact zero
+            ns.k[ns.nk] = (*vars[0].k)[j].get();
+            ns.c[ns.nk++] = (float)(h * a[j]);
+          }
         ns.cself = (float)(h * a[cross ? 0 : st]);
         ns.out = fused->xn.get();
         ns.N = fused->N;
         world_->eval_rhs_all(vars, st, s, st > 0, 0.0, &ns);
+        if (trade_x0) {
+          std::swap(fused->m, fused->x0);
+          trade_x0 = false;
+        }
         if (cross) {
           next_valid_ = true;
           next_h_ = h;
+        } else if (last) {
+          std::swap(fused->m, fused->xn);
+          vars[0].x = fused->m.get();
         } else {
           have_next = true;
         }
@@ -1984,7 +1998,7 @@ void TimeSolver::step() {
       nrhs += (long long)vars.size();
     }
     time = t0 + h;
-    if (!tb.fsal) combine(tb.w1, S, h, -1);
+    if (!tb.fsal && !fused) combine(tb.w1, S, h, -1);
     ++nsteps;
     if (!adaptive) break;
     double err = 0.0;
