@@ -854,6 +854,42 @@ __global__ void __launch_bounds__(XinvCfg<L2>::THREADS)
   xinv_body<L2>(d, A, geom, h, tw, xcd_remap(blockIdx.x, gridDim.x));
 }
 
+// ---------------------------------------------------------------- direct sum (small grids)
+
+__device__ __forceinline__ void direct_body(const DirectDesc& D, const DirectSource& S, float* __restrict__ h,
+                                            int blk) {
+  extern __shared__ float2 lds[];
+  float* src = reinterpret_cast<float*>(lds);
+  direct_stage(D, S, src);
+  float* red = src + direct_lds_floats(D.nb, D.rows);
+  int i;
+  float3 v;
+  if (!(D.K2 ? direct_sum<false>(D, src, red, blk, i, v) : direct_sum<true>(D, src, red, blk, i, v))) return;
+  if (S.geom && !S.geom[i]) v = f3(0.f, 0.f, 0.f);
+  h[i] = v.x;
+  h[S.cs + i] = v.y;
+  h[2 * S.cs + i] = v.z;
+}
+
+__global__ void __launch_bounds__(1024) k_direct(DirectDesc D, DirectSource S, float* __restrict__ h) {
+  direct_body(D, S, h, blockIdx.x);
+}
+
+// The direct sum's kernel table from the FP64 octant in[c][z][y][x].
+__global__ void k_direct_table(const double* __restrict__ in, int nx, int rows, int row4, double pref,
+                               float4* __restrict__ k4, float2* __restrict__ k2) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= rows * 2 * row4) return;
+  const int r = e / (2 * row4), dx = e - r * 2 * row4 - row4, x = dx < 0 ? -dx : dx;
+  const size_t n = (size_t)nx * rows, i = (size_t)r * nx + x;
+  const double sx = dx < 0 ? -pref : pref;
+  float v[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (x < nx)
+    for (int c = 0; c < 6; ++c) v[c] = (float)((c == 3 || c == 4 ? sx : pref) * in[c * n + i]);
+  k4[e] = make_float4(v[0], v[1], v[2], v[3]);
+  if (k2) k2[e] = make_float2(v[4], v[5]);
+}
+
 // ------------------------------------------------ kernel spectrum (FP64)
 
 __global__ void k_newell_octant(double* __restrict__ out, int nx, int ny, int nz, double cx, double cy, double cz,
@@ -1371,6 +1407,22 @@ DemagPlan::DemagPlan(const DemagGeometry& g) : g_(g) {
   build_kernel(nullptr);
 }
 
+namespace {
+// Grids whose field is summed directly: those where the one launch beats the
+// FFT passes.  Single layers (5 products a pair) up to 4096 cells: 12.3 against
+// 14.0 us there, 5.4 against 12.8 at 960.  More layers (9 products a pair, and
+// five passes on the other side) up to 3584: 12.1 against 19.4 us at 2550.  At
+// 8192 cells the sum takes two to three times the passes.  A batch keeps the
+// passes for every member: it is bound by throughput, where N^2 products lose
+// (256 members of up to 65536 cells: 172 against 91 ms with the members below
+// these limits summed).  Grids of up to 640 cells keep the passes too, so that
+// such a magnet's own steps round as its steps in a batch do.
+bool direct_rule(int nx, int ny, int nz) {
+  const long long n = (long long)nx * ny * nz;
+  return n > 640 && n <= (nz == 1 ? 4096 : 3584) && (long long)ny * nz * ((nx + 3) / 4) <= 3072;
+}
+}  // namespace
+
 void DemagPlan::build_kernel(hipStream_t s) {
   const int nx = g_.n[0], ny = g_.n[1], nz = g_.n[2];
   DeviceArray<double> oct((size_t)6 * N_);
@@ -1378,6 +1430,25 @@ void DemagPlan::build_kernel(hipStream_t s) {
                                                  g_.mastergrid[0], g_.mastergrid[1], g_.mastergrid[2], g_.pbc[0],
                                                  g_.pbc[1], g_.pbc[2]);
   checkLaunch("k_newell_octant");
+  direct_ = direct_rule(nx, ny, nz);
+  if (direct_) {
+    DirectDesc& D = direct_desc_;
+    D.nx = nx; D.ny = ny; D.nz = nz;
+    D.nb = (nx + 3) / 4;
+    D.rows = ny * nz;
+    auto magic = [](int d) { return (unsigned)((1ull << 32) / (unsigned)d + 1); };
+    D.mag_nb = magic(D.nb);
+    D.mag_ny = magic(ny);
+    direct_shape(D);
+    const size_t n = (size_t)D.rows * 8 * D.nb;
+    direct_k4_.allocate(n);
+    if (nz > 1) direct_k2_.allocate(n);
+    D.K4 = direct_k4_.get();
+    D.K2 = direct_k2_.get();
+    k_direct_table<<<grid_for((long long)n), BLOCK, 0, s>>>(oct.get(), nx, D.rows, 4 * D.nb, -MU0, direct_k4_.get(),
+                                                            direct_k2_.get());
+    checkLaunch("k_direct_table");
+  }
   DeviceArray<double> ct[3], st[3];
   for (int a = 0; a < 3; ++a) make_trig(ct[a], st[a], K_[a]);
   // odd components per axis: x: xy(3), xz(4); y: xy(3), yz(5); z: xz(4), yz(5)
@@ -1477,6 +1548,14 @@ void DemagPlan::exec_combine(const float* x0, const Combo& co, float* x, PS msat
 
 void DemagPlan::run(float2* A, float2* B, const float* m, PS msat, const uint8_t* geom, float* h, hipStream_t s,
                     Profiler* prof, const float* m2, PS msat2, const StageIn* in) {
+  if (direct_ && !in) {
+    Timed t(prof, "k_direct", direct_bytes() + (m2 ? 12.0 * N_ : 0.0), s);
+    const DirectDesc& D = direct_desc_;
+    const DirectLaunch L = direct_launch(D);
+    k_direct<<<L.blocks, L.threads, L.shm, s>>>(D, DirectSource{m, msat, m2, msat2, geom, (size_t)N_}, h);
+    checkLaunch("k_direct");
+    return;
+  }
   DD d;
   d.nx = g_.n[0]; d.ny = g_.n[1]; d.nz = g_.n[2];
   d.Kx = K_[0]; d.Ky = K_[1]; d.Kz = K_[2];
@@ -1674,6 +1753,10 @@ double DemagPlan::pass_bytes(int i) const {
   const double v[5] = {12 * N + xa, xa + yb, 2 * yb + t, yb + xa, xa + 12 * N};
   return v[i];
 }
+
+// The source read, the kernel's octant read (xx, yy, zz, xy; with layers xz
+// and yz too) and the field written, once each.
+double DemagPlan::direct_bytes() const { return (24.0 + (is2d() ? 16.0 : 24.0)) * N_; }
 
 double DemagPlan::algorithmic_bytes() const {
   double b = 0.0;

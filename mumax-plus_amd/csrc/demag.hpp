@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "demag_direct.hpp"
 #include "profiler.hpp"
 #include "rk.hpp"
 
@@ -52,6 +53,11 @@ class DemagPlan {
   size_t workspace_bytes() const;
   // Allocates A and B if the plan does not hold them yet.
   void ensure_workspace();
+  // Whether exec sums the real-space kernel directly (small grids; one
+  // launch, no intermediates), and the description of that sum.
+  bool direct() const { return direct_; }
+  const DirectDesc& direct_desc() const { return direct_desc_; }
+  double direct_bytes() const;  // algorithmic HBM bytes of the direct sum
   // Pass names and algorithmic HBM bytes per pass.
   int npasses() const { return is2d() ? 3 : 5; }
   const char* pass_name(int i) const;
@@ -88,6 +94,10 @@ class DemagPlan {
   DeviceArray<float2> A_, B_;
   DeviceArray<float> T_;
   DeviceArray<float2> tw_[3];
+  bool direct_ = false;
+  DirectDesc direct_desc_{};
+  DeviceArray<float4> direct_k4_;
+  DeviceArray<float2> direct_k2_;
 };
 
 // Demag of many independent magnets at once, each with its own plan.  The

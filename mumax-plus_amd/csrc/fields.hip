@@ -25,6 +25,7 @@
 
 #include "field_cell.hpp"
 
+#include "demag_direct.hpp"
 #include "philox.hpp"
 
 namespace mpa {
@@ -59,17 +60,15 @@ __device__ __forceinline__ float3 normalized3(float3 v) {
   return v / n;
 }
 
+// Cell idx (< ncell) with any parameters; hdem(idx) gives its demag field.
 // UNI: every parameter is uniform, so each lookup is the scalar and the
 // harmonic mean of a cell and its neighbour is the value itself.  NK >= 0:
 // the cell also writes the next Runge-Kutta stage state (nx, NK derivatives
 // from memory and the one just computed; x0 == nullptr: the cell's state).
-template <bool UNI, int NK = -2>
-__device__ __forceinline__ void field_body(const FMDesc& d, const float* __restrict__ m,
-                                           const float* __restrict__ hdemag, float* __restrict__ out, int mode,
-                                           int bid, const NextStage* nx = nullptr) {
-  const int idx = bid * BLOCK + threadIdx.x;
+template <bool UNI, int NK, class HDem>
+__device__ __forceinline__ void field_cell(const FMDesc& d, const float* __restrict__ m, const HDem& hdemag,
+                                           float* __restrict__ out, int mode, int idx, const NextStage* nx) {
   const int N = d.ncell;
-  if (idx >= N) return;
   auto S = [&](const PS& p, int i) { return UNI ? p.v : p.at(i); };
   auto V = [&](const PV& p, int i) { return UNI ? make_float3(p.x, p.y, p.z) : p.at(i, N); };
   auto HM = [&](float u, float v) { return UNI ? u : harmonic_mean(u, v); };
@@ -332,7 +331,7 @@ __device__ __forceinline__ void field_body(const FMDesc& d, const float* __restr
     if (d.hstray) hext = hext + load3(d.hstray, idx, N);
   }
   float3 hdem = f3(0.f, 0.f, 0.f);
-  if (d.terms & TERM_DEMAG) hdem = load3(hdemag, idx, N);
+  if (d.terms & TERM_DEMAG) hdem = hdemag(idx);
 
   if (mode == MODE_EDENS) {
     edens += -0.5f * ms * dot3(mc, hex);
@@ -433,6 +432,16 @@ __device__ __forceinline__ void field_body(const FMDesc& d, const float* __restr
   out[N + idx] = r.y;
   out[2 * N + idx] = r.z;
   if constexpr (NK >= 0) nx->template apply<NK>(idx, mc, r, true);
+}
+
+// One cell per thread, the demag field from memory.
+template <bool UNI, int NK = -2>
+__device__ __forceinline__ void field_body(const FMDesc& d, const float* __restrict__ m,
+                                           const float* __restrict__ hdemag, float* __restrict__ out, int mode,
+                                           int bid, const NextStage* nx = nullptr) {
+  const int idx = bid * BLOCK + threadIdx.x;
+  if (idx >= d.ncell) return;
+  field_cell<UNI, NK>(d, m, [&](int i) { return load3(hdemag, i, d.ncell); }, out, mode, idx, nx);
 }
 
 template <bool UNI>
@@ -547,6 +556,35 @@ __global__ void __launch_bounds__(BLOCK) k_field_uniform(FMDesc d, FMUniform u, 
         });
       else field_uniform_cell(d, u, m, hd, out, mode, x, y, z, N);
     }
+  }
+}
+
+// A small magnet's whole evaluation in one launch: the demag field summed
+// directly (demag_direct.hpp), and on the four lanes that hold a strip's
+// fields the field, the torque and (NK >= 0) the next stage state of its
+// cells.  KIND 0: uniform path; 1, 2: per-cell kernel with uniform / any
+// parameters.  Latency-bound: 4 launches of 5 us become one.
+template <int KIND, int NK>
+__global__ void __launch_bounds__(1024) k_field_direct(DirectDesc D, FMDesc d, FMUniform u,
+                                                       const float* __restrict__ m, float* __restrict__ out, int mode,
+                                                       NextStage next) {
+  extern __shared__ __align__(16) float dlds[];
+  direct_stage(D, DirectSource{m, d.msat, nullptr, PS{nullptr, 0.f}, d.geom, (size_t)d.ncell}, dlds);
+  float* red = dlds + direct_lds_floats(D.nb, D.rows);
+  int idx;
+  float3 h;
+  if (!(D.K2 ? direct_sum<false>(D, dlds, red, blockIdx.x, idx, h) : direct_sum<true>(D, dlds, red, blockIdx.x, idx, h)))
+    return;
+  auto hd = [&](int) { return h; };
+  if constexpr (KIND == 0) {
+    const int x = idx % d.nx, yz = idx / d.nx, y = yz % d.ny, z = yz / d.ny;
+    if constexpr (NK >= 0)
+      field_uniform_cell(d, u, m, hd, out, mode, x, y, z, d.ncell, [&](int i, float3 mc, float3 r, bool in) {
+        next.template apply<NK>(i, mc, r, in);
+      });
+    else field_uniform_cell(d, u, m, hd, out, mode, x, y, z, d.ncell);
+  } else {
+    field_cell<KIND == 1, NK>(d, m, hd, out, mode, idx, &next);
   }
 }
 
@@ -1109,6 +1147,36 @@ void launch_field_next(const FMDesc& d, const float* m, const float* hdemag, flo
   }
 #undef MPA_FIELD_NEXT
   checkLaunch("k_field_next");
+}
+
+void launch_field_direct(const DirectDesc& D, const FMDesc& d, const float* m, float* out, FieldMode mode,
+                         const NextStage* next, hipStream_t s) {
+  if (mode != MODE_LLG && mode != MODE_DAMPING) throw Error(MPA_ERR_RUNTIME, "launch_field_direct: torques only");
+  if (!(d.terms & TERM_DEMAG) || d.sublattice) throw Error(MPA_ERR_RUNTIME, "launch_field_direct: no demag field");
+  if (next && (!field_next_fusable(d, mode) || next->nk < 0 || next->nk > 5 || !next->out || next->out == m ||
+               next->out == out || next->out == next->x0))
+    throw Error(MPA_ERR_RUNTIME, "launch_field_direct: bad stage combination");
+  const int kind = all_uniform(d) ? 0 : (params_uniform(d) ? 1 : 2);
+  const FMUniform u = kind == 0 ? make_uniform(d) : FMUniform{};
+  const NextStage ns = next ? *next : NextStage{};
+  const DirectLaunch L = direct_launch(D);
+#define MPA_DIRECT(K)                                                                                              \
+  switch (kind) {                                                                                                  \
+    case 0: k_field_direct<0, K><<<L.blocks, L.threads, L.shm, s>>>(D, d, u, m, out, (int)mode, ns); break;        \
+    case 1: k_field_direct<1, K><<<L.blocks, L.threads, L.shm, s>>>(D, d, u, m, out, (int)mode, ns); break;        \
+    default: k_field_direct<2, K><<<L.blocks, L.threads, L.shm, s>>>(D, d, u, m, out, (int)mode, ns); break;       \
+  }
+  switch (next ? ns.nk : -2) {
+    case 0: MPA_DIRECT(0) break;
+    case 1: MPA_DIRECT(1) break;
+    case 2: MPA_DIRECT(2) break;
+    case 3: MPA_DIRECT(3) break;
+    case 4: MPA_DIRECT(4) break;
+    case 5: MPA_DIRECT(5) break;
+    default: MPA_DIRECT(-2) break;
+  }
+#undef MPA_DIRECT
+  checkLaunch("k_field_direct");
 }
 
 void launch_field(const FMDesc& d, const float* m, const float* hdemag, float* out, FieldMode mode, hipStream_t s) {

@@ -140,6 +140,13 @@ bool field_next_fusable(const FMDesc& d, FieldMode mode);
 void launch_field_next(const FMDesc& d, const float* m, const float* hdemag, float* out, FieldMode mode,
                        const NextStage& next, hipStream_t s);
 
+// The torque (MODE_LLG or MODE_DAMPING) of a magnet whose demag plan sums
+// directly (DemagPlan::direct), demag field included, in one launch; with
+// `next` also the next stage state, for field_next_fusable magnets.
+struct DirectDesc;
+void launch_field_direct(const DirectDesc& D, const FMDesc& d, const float* m, float* out, FieldMode mode,
+                         const NextStage* next, hipStream_t s);
+
 // The tile-schedule autotuner's record of the uniform field kernel (z planes
 // per workgroup chosen per grid size and kernel variant when FMDesc.tile_zc
 // is -1): one line per grid, the choice and the microseconds per launch of

@@ -938,10 +938,18 @@ FMDesc Ferromagnet::rhs_desc(unsigned terms, double noise_dt) {
 }
 
 void Ferromagnet::eval_rhs(float* out, hipStream_t s, bool prepared, FieldMode mode, double noise_dt,
-                           const NextStage* next) {
+                           const NextStage* next, bool demag_ready) {
   const unsigned terms = active_terms();
   Profiler* prof = &world->prof;
-  if (!prepared) prepare(terms, s, prof);
+  const bool direct = !demag_ready && !host && (terms & TERM_DEMAG) && demag().direct();
+  if (!prepared) prepare(direct ? terms & ~TERM_DEMAG : terms, s, prof);
+  if (direct) {
+    // the demag sum reads the magnetisation and writes no field
+    const double bytes = 24.0 * N + (next ? 12.0 * N * ((next->x0 ? 1 : 0) + next->nk + 1) : 0.0);
+    Timed t(prof, next ? "k_field_next" : "k_field", bytes, s);
+    launch_field_direct(demag().direct_desc(), rhs_desc(terms, noise_dt), m.get(), out, mode, next, s);
+    return;
+  }
   if (next) {
     // plus the combination: read x0 (unless it is the cell's own state) and
     // nk derivatives, write the next stage state
@@ -953,6 +961,8 @@ void Ferromagnet::eval_rhs(float* out, hipStream_t s, bool prepared, FieldMode m
   Timed t(prof, "k_field", rhs_bytes(terms), s);
   launch_field(rhs_desc(terms, noise_dt), m.get(), demag_field(), out, mode, s);
 }
+
+bool Ferromagnet::direct_rhs() { return !host && (active_terms() & TERM_DEMAG) && demag().direct(); }
 
 bool Ferromagnet::next_fusable() {
   if (host || el.enabled) return false;
@@ -1453,9 +1463,9 @@ void World::eval_rhs_all(const std::vector<StateVar>& vars, int stage, hipStream
         if (stage_in)
           fm->demag().exec_combine(stage_in->x0, stage_in->co, fm->m.get(), fm->param("msat").ps(), fm->geom_ptr(),
                                    fm->hdemag.get(), s, &prof);
-        else if (t & TERM_DEMAG)
+        else if ((t & TERM_DEMAG) && !fm->direct_rhs())
           fm->demag().exec(fm->m.get(), fm->param("msat").ps(), fm->geom_ptr(), fm->hdemag.get(), s, &prof);
-        fm->eval_rhs(out, s, true, mode, noise_dt, next);
+        fm->eval_rhs(out, s, true, mode, noise_dt, next, stage_in != nullptr);
       }
     } else if (sv.kind == StateVar::DISP) {
       // du/dt = v (elastodynamics.cu:93-96); a stage's combination may have

@@ -249,14 +249,20 @@ class Ferromagnet : public MagnetCore {
 
   // out (device, 3N) = torque of the current magnetisation (the LLG torque,
   // or the damping-only torque of a relaxation).  With prepared, the demag
-  // field and strain are taken as already computed.
+  // field and strain are taken as already computed; a demag field that is
+  // summed directly is formed in the same launch, unless demag_ready tells
+  // that hdemag holds it.
   // noise_dt > 0: add the thermal field of the step in progress divided by
   // sqrt(noise_dt) (the stepper's noise term).
   void eval_rhs(float* out, hipStream_t s, bool prepared = false, FieldMode mode = MODE_LLG, double noise_dt = 0.0,
-                const NextStage* next = nullptr);
+                const NextStage* next = nullptr, bool demag_ready = false);
   // The right-hand side can also write the next stage state in the same
   // launch (the uniform-parameter LLG path of an independent magnet).
   bool next_fusable();
+  // Whether the right-hand side is one launch with the demag field summed
+  // directly (launch_field_direct): the demag plan's own exec is then not
+  // needed, and hdemag is not written.
+  bool direct_rhs();
   double rhs_bytes(unsigned terms);
   FMDesc rhs_desc(unsigned terms, double noise_dt);
   int eval_quantity(const std::string& q, float* host, hipStream_t s);

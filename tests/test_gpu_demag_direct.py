@@ -1,0 +1,86 @@
+"""The direct demag sum of small grids, and the one-launch evaluation on it.
+
+Grids at the edges of the strips (four x cells), of the wavefronts per strip
+and of the rule that chooses the sum, against the FP64 oracle: field error at
+most 4e-7 of the largest field (FP32 kernel and products, short chains).  The
+same magnets' torque, which one launch forms with the field, against the
+torque formed from the demag field in memory by the per-cell kernel.
+"""
+
+import numpy as np
+import pytest
+
+from helpers import make_pair, random_unit
+from oracle import demag as odemag
+
+import mumaxplus as mp
+
+pytestmark = pytest.mark.gpu
+
+# 641 cells and more are summed; the last three lie on the other side of the
+# rule.  No axis is longer than 350 cells: the FP64 tensor's own cancellation
+# (27 terms of r^3 2^-53 / (4 pi) at r cells) is 1e-8 there, but 8e-8 an entry
+# at 700, which the oracle and the device round differently.
+SIZES = [(214, 3, 1), (3, 214, 1), (2, 2, 161), (64, 64, 1), (257, 3, 1), (128, 32, 1), (43, 15, 1), (2, 350, 3),
+         (33, 9, 4), (16, 16, 14), (64, 65, 1), (32, 16, 8), (32, 20, 1)]
+
+
+def _grid(size):
+    nx, ny, nz = size
+    rng = np.random.default_rng(nx + 7 * ny + 31 * nz)
+    m = random_unit(rng, (nz, ny, nx)).astype(np.float32)
+    return rng, m
+
+
+@pytest.mark.parametrize("size", SIZES)
+def test_field(size):
+    rng, m = _grid(size)
+    nx, ny, nz = size
+    cs = (3e-9, 2e-9, 4e-9)
+    world = mp.World(cs)
+    geom = rng.random((nz, ny, nx)) > 0.2 if nx * ny * nz > 20 else None
+    mag = mp.Ferromagnet(world, mp.Grid(size), geometry=geom)
+    ms = (8e5 * rng.uniform(0.5, 1.5, (nz, ny, nx))).astype(np.float32)
+    mag.msat = ms
+    mag.magnetization = m
+    want = odemag.demag_fft(mag.magnetization.get().astype(float), ms.astype(float), world.cellsize, geom)
+    got = mag.demag_field()
+    assert np.abs(got - want).max() <= 4e-7 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("pbc", [(1, 0, 0), (2, 1, 0)])
+def test_periodic(pbc):
+    size = (38, 11, 2)
+    _, m = _grid(size)
+    cs = (3e-9, 2e-9, 4e-9)
+    box = tuple(n if p else 0 for n, p in zip(size, pbc))
+    world = mp.World(cs, mastergrid=mp.Grid(box), pbc_repetitions=pbc)
+    mag = mp.Ferromagnet(world, mp.Grid(size))
+    mag.msat = 8e5
+    mag.magnetization = m
+    want = odemag.demag_fft(mag.magnetization.get().astype(float), 8e5, world.cellsize, None, box, pbc)
+    assert np.abs(mag.demag_field() - want).max() <= 4e-7 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("size", [(51, 13, 1), (64, 64, 1), (33, 9, 4), (16, 16, 14)])
+@pytest.mark.parametrize("kind", ["uniform", "uniform parameters", "per cell"])
+def test_stepped_torque(size, kind):
+    """One fixed Heun step takes two one-launch evaluations; the oracle's step is the reference."""
+    rng, m = _grid(size)
+    nx, ny, nz = size
+    p = {"msat": 8e5, "aex": 1.3e-11, "alpha": 0.05, "ku1": 3e5, "anisU": (0, 0.6, 0.8)}
+    if kind == "uniform parameters":
+        p.update(jcur=(1e12, 0, 0), xi=0.1, pol=0.5)
+    if kind == "per cell":
+        p["ku1"] = (3e5 * rng.uniform(0.5, 1.5, (nz, ny, nx))).astype(np.float32)
+    world, mag, ow, om = make_pair(size, (3e-9, 2e-9, 4e-9), p, m, geometry=rng.random((nz, ny, nx)) > 0.2)
+    for ts in (world.timesolver, ow.solver):
+        ts.set_method("Heun")
+    world.timesolver.adaptive_timestep, world.timesolver.timestep = False, 2e-14
+    ow.solver.adaptive, ow.solver.dt = False, 2e-14
+    m0 = mag.magnetization.get().astype(float)
+    world.timesolver.steps(1)
+    ow.solver.steps(1)
+    dm, want = mag.magnetization.get() - m0, om.m - m0
+    # the step moves m by up to a few percent: its error is that of m (2^-24) over the move
+    assert np.abs(dm - want).max() <= 1e-5 * np.abs(want).max() + 1.5e-7
