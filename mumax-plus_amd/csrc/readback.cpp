@@ -1,0 +1,133 @@
+// A copy into pageable memory runs at 9 GB/s: the driver bounces it through a
+// pinned buffer with one thread, and that thread also takes every page fault
+// of a freshly allocated destination.  Here several host threads share the
+// bytes out in chunks; each moves its chunks through two pinned buffers of its
+// own, so the device's copies, the memory copies and the page faults of
+// different chunks overlap.
+#include "readback.hpp"
+
+#include <algorithm>
+#include <cstring>
+#include <exception>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "common.hpp"
+
+namespace mpa {
+
+namespace {
+
+constexpr size_t CHUNK = (size_t)1 << 20;
+constexpr int THREADS = 8;
+constexpr size_t MIN_BYTES = (size_t)3 << 20;  // below, one thread's copy is as fast
+
+struct Lane {
+  char* pin[2] = {nullptr, nullptr};
+  hipEvent_t ev[2] = {nullptr, nullptr};
+};
+
+// One set of buffers (16 MiB pinned) per process and one device; a second
+// reader at the same time, or one on another device, takes the plain copy.
+std::mutex mu;       // held for the length of a read
+std::mutex count_mu;
+int worlds = 0;
+int device = -1;
+Lane lanes[THREADS];
+
+void drop() {
+  for (Lane& l : lanes)
+    for (int b = 0; b < 2; ++b) {
+      if (l.ev[b]) (void)hipEventDestroy(l.ev[b]);
+      if (l.pin[b]) (void)hipHostFree(l.pin[b]);
+      l.ev[b] = nullptr;
+      l.pin[b] = nullptr;
+    }
+  device = -1;
+}
+
+void plain(void* host, const void* dev, size_t bytes, hipStream_t s) {
+  HIP_CHECK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s));
+  HIP_CHECK(hipStreamSynchronize(s));
+}
+
+bool ready() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  if (device == dev) return true;
+  if (device >= 0) return false;
+  for (Lane& l : lanes)
+    for (int b = 0; b < 2; ++b)
+      if (hipHostMalloc(reinterpret_cast<void**>(&l.pin[b]), CHUNK, hipHostMallocDefault) != hipSuccess ||
+          hipEventCreateWithFlags(&l.ev[b], hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        drop();
+        return false;
+      }
+  device = dev;
+  return true;
+}
+
+}  // namespace
+
+void readback_retain() {
+  std::lock_guard<std::mutex> lk(count_mu);
+  ++worlds;
+}
+
+void readback_release() {
+  std::lock_guard<std::mutex> lk(count_mu);
+  if (--worlds > 0) return;
+  std::lock_guard<std::mutex> lk2(mu);
+  drop();
+}
+
+void read_back(void* host, const void* dev, size_t bytes, hipStream_t s) {
+  std::unique_lock<std::mutex> lk(mu, std::defer_lock);
+  if (bytes < MIN_BYTES || !lk.try_lock() || !ready()) {
+    plain(host, dev, bytes, s);
+    return;
+  }
+  const size_t n = (bytes + CHUNK - 1) / CHUNK;
+  const int T = (int)std::min<size_t>(THREADS, n);
+  std::exception_ptr failed[THREADS];
+  auto work = [&](int t) {
+    try {
+      HIP_CHECK(hipSetDevice(device));
+      Lane& l = lanes[t];
+      auto issue = [&](size_t c, int b) {
+        const size_t off = c * CHUNK, len = std::min(CHUNK, bytes - off);
+        HIP_CHECK(hipMemcpyAsync(l.pin[b], static_cast<const char*>(dev) + off, len, hipMemcpyDeviceToHost, s));
+        HIP_CHECK(hipEventRecord(l.ev[b], s));
+      };
+      int b = 0;
+      if ((size_t)t < n) issue(t, 0);
+      for (size_t c = t; c < n; c += T, b ^= 1) {
+        if (c + T < n) issue(c + T, b ^ 1);
+        HIP_CHECK(hipEventSynchronize(l.ev[b]));
+        const size_t off = c * CHUNK;
+        std::memcpy(static_cast<char*>(host) + off, l.pin[b], std::min(CHUNK, bytes - off));
+      }
+    } catch (...) {
+      failed[t] = std::current_exception();
+    }
+  };
+  std::vector<std::thread> pool;
+  pool.reserve(T);
+  int started = 1;
+  try {
+    for (; started < T; ++started) pool.emplace_back(work, started);
+  } catch (...) {
+    // no more threads: the started ones end, and their shares are copied again below
+  }
+  work(0);
+  for (std::thread& th : pool) th.join();
+  // every queued copy ends before the buffers are used again
+  HIP_CHECK(hipStreamSynchronize(s));
+  for (int t = 0; t < started; ++t)
+    if (failed[t]) std::rethrow_exception(failed[t]);
+  if (started < T) plain(host, dev, bytes, s);
+}
+
+}  // namespace mpa

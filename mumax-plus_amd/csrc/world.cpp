@@ -1,5 +1,6 @@
 // Host object model and the Runge-Kutta time stepper.
 #include "world.hpp"
+#include "readback.hpp"
 
 #include <algorithm>
 #include <array>
@@ -457,8 +458,7 @@ void MagnetCore::get_variable(const std::string& which, float* host, hipStream_t
   const DeviceArray<float>* src =
       which == "elastic_displacement" ? &el.u : (which == "elastic_velocity" ? &el.v : nullptr);
   if (!src) throw Error(MPA_ERR_INVALID, "unknown variable '" + which + "'");
-  HIP_CHECK(hipMemcpyAsync(host, src->get(), (size_t)3 * N * sizeof(float), hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipStreamSynchronize(s));
+  read_back(host, src->get(), (size_t)3 * N * sizeof(float), s);
 }
 
 namespace {
@@ -1154,8 +1154,7 @@ const float* Ferromagnet::eval_device(const std::string& q, hipStream_t s, int* 
 int Ferromagnet::eval_quantity(const std::string& q, float* host_out, hipStream_t s) {
   int nc = 0;
   const float* dev = eval_device(q, s, &nc);
-  HIP_CHECK(hipMemcpyAsync(host_out, dev, (size_t)nc * N * sizeof(float), hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipStreamSynchronize(s));
+  read_back(host_out, dev, (size_t)nc * N * sizeof(float), s);
   return nc;
 }
 
@@ -1229,8 +1228,7 @@ void Ferromagnet::set_magnetization(const float* host_in, long long count, hipSt
 }
 
 void Ferromagnet::get_magnetization(float* host_out, hipStream_t s) {
-  HIP_CHECK(hipMemcpyAsync(host_out, m.get(), (size_t)3 * N * sizeof(float), hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipStreamSynchronize(s));
+  read_back(host_out, m.get(), (size_t)3 * N * sizeof(float), s);
 }
 
 // ------------------------------------------------------------ Antiferromagnet
@@ -1339,8 +1337,7 @@ double Antiferromagnet::scalar_quantity(const std::string& q, hipStream_t s) {
 int Antiferromagnet::eval_quantity(const std::string& q, float* host_out, hipStream_t s) {
   int nc = 0;
   const float* dev = eval_device(q, s, &nc);
-  HIP_CHECK(hipMemcpyAsync(host_out, dev, (size_t)nc * N * sizeof(float), hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipStreamSynchronize(s));
+  read_back(host_out, dev, (size_t)nc * N * sizeof(float), s);
   return nc;
 }
 
@@ -2082,6 +2079,7 @@ World::World(const double cs[3], const int mg_size[3], const int mg_origin[3], c
   HIP_CHECK(hipStreamCreateWithFlags(&stream3, hipStreamNonBlocking));
   for (hipEvent_t* e : {&ev_fork, &ev_strain, &ev_local, &ev_join, &ev_join3})
     HIP_CHECK(hipEventCreateWithFlags(e, hipEventDisableTiming));
+  readback_retain();
 }
 
 World::~World() {
@@ -2092,6 +2090,7 @@ World::~World() {
   if (stream3) (void)hipStreamDestroy(stream3);
   if (stream2) (void)hipStreamDestroy(stream2);
   if (stream) (void)hipStreamDestroy(stream);
+  readback_release();
 }
 
 // World::checkPbcRepetitions / checkPbcCompatibility (src/core/world.cpp:62-76)
