@@ -598,7 +598,8 @@ void Batch::build_persist() {
   std::vector<bk::Phase> ph;
   // the demag passes as phases: the two groups' chains side by side
   // (members with a z transform: xfwd, yfwd, zpass, yinv, xinv; single
-  // layers: xfwd, ypass2d, xinv, whose x inverse shares the z pass's phase)
+  // layers: xfwd, ypass2d, xinv, whose x inverse shares the z pass's phase;
+  // the yz pass of few layers shares the y inverse's)
   bk::Phase dph[5];
   for (auto& d : dph) {
     d = bk::Phase{};
@@ -607,8 +608,8 @@ void Batch::build_persist() {
   size_t shm = 0;
   if (demag_) {
     for (const DemagBatch::PassTable& t : demag_->pass_tables()) {
-      static const int slot0[6] = {0, 1, 2, 3, -1, 4};
-      static const int slot1[6] = {0, -1, -1, -1, 1, 2};
+      static const int slot0[7] = {0, 1, 2, 3, -1, 4, 3};
+      static const int slot1[7] = {0, -1, -1, -1, 1, 2, -1};
       const int slot = t.group == 0 ? slot0[t.pass] : slot1[t.pass];
       if (slot < 0) throw Error(MPA_ERR_RUNTIME, "batch: unexpected demag pass");
       bk::Phase& d = dph[slot];

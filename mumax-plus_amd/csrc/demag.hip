@@ -100,6 +100,7 @@ struct BSeg {
   float2* B;
   const float* T;
   const float2* tw[3];
+  const float2* Tz;  // few layers (pass 6)
   int first;
 };
 
@@ -854,6 +855,175 @@ __global__ void __launch_bounds__(XinvCfg<L2>::THREADS)
   xinv_body<L2>(d, A, geom, h, tw, xcd_remap(blockIdx.x, gridDim.x));
 }
 
+// ---------------------------------------------------------------- y and z of few layers
+
+// Two to eight layers: the passes between the x transforms as one.  A block
+// takes one kx: it transforms the 3 Nz y-lines of that kx into LDS, forms for
+// every ky the layers' convolution along z directly from the kernel's (x, y)
+// spectrum at each layer distance,
+//   h_a(z) = sum_z' sum_b K_ab(z - z') m_b(z'),
+// in place of a padded z transform, and transforms back.  So B (twice A's
+// size, written and read twice) is gone, the products are 9 Nz^2 against the
+// two transforms of 8 or 16 points and the tensor product, and two launches
+// go.  The components odd in z (xz, yz) have one odd axis left in the (x, y)
+// transform: their spectrum is -i times a real sine sum.
+// Table Tz[kx][dz][3][Hy] of float2: (xx, yy), (zz, xy), (xz, yz): consecutive
+// ky lie side by side, so a wavefront's loads are whole lines.
+constexpr int FEW_MAX = 8;
+
+template <int L2, int TH>
+struct YzCfg {
+  using C = Line<L2>;
+  static constexpr int LB = TH / C::T;  // lines transformed at a time
+  static constexpr int THREADS = LB * C::T;
+  // transforms and the column reads take consecutive elements of a line
+  static constexpr int LP = C::stride(C::fft_target());
+  // lines of several wavefronts: one more buffer for the groups past the last line
+  static size_t shm(int nz) { return (size_t)(3 * nz + (C::T > 64 ? 1 : 0)) * LP * sizeof(float2); }
+};
+
+template <int NZ, int L2, class K>
+__device__ __forceinline__ void yz_convolve(const DD& d, float2* lds, const float2* __restrict__ Tz, int kx) {
+  using C = Line<L2>;
+  const float2* row = Tz + (size_t)kx * NZ * 3 * d.Hy;
+  for (int ky = threadIdx.x; ky < C::L; ky += K::THREADS) {
+    const bool up = ky > (C::L >> 1);  // mirrored: the components odd in y change sign
+    const int kh = up ? C::L - ky : ky;
+    const float sy = up ? -1.f : 1.f;
+    float2* col = lds + iopad<L2>(ky);
+    float2 m[3][NZ], h[3][NZ];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int z = 0; z < NZ; ++z) {
+        m[c][z] = col[(c * NZ + z) * K::LP];
+        h[c][z] = make_float2(0.f, 0.f);
+      }
+#pragma unroll
+    for (int dz = 0; dz < NZ; ++dz) {
+      const float2 a = row[(dz * 3 + 0) * d.Hy + kh], b = row[(dz * 3 + 1) * d.Hy + kh];
+      const float2 e = row[(dz * 3 + 2) * d.Hy + kh];
+      const float xx = a.x, yy = a.y, zz = b.x, xy = sy * b.y, xz = e.x, yz = sy * e.y;
+#pragma unroll
+      for (int z = 0; z < NZ; ++z)
+#pragma unroll
+        for (int up_z = 0; up_z < 2; ++up_z) {
+          const int q = up_z ? z + dz : z - dz;  // source layer
+          if (q < 0 || q >= NZ || (dz == 0 && up_z)) continue;
+          const float2 mx = m[0][q], my = m[1][q], mz = m[2][q];
+          h[0][z].x += xx * mx.x + xy * my.x;
+          h[0][z].y += xx * mx.y + xy * my.y;
+          h[1][z].x += xy * mx.x + yy * my.x;
+          h[1][z].y += xy * mx.y + yy * my.y;
+          h[2][z].x += zz * mz.x;
+          h[2][z].y += zz * mz.y;
+          if (dz != 0) {
+            // -i s (xz, yz), s the sign of z - q
+            const float sxz = up_z ? -xz : xz, syz = up_z ? -yz : yz;
+            h[0][z].x += sxz * mz.y;
+            h[0][z].y -= sxz * mz.x;
+            h[1][z].x += syz * mz.y;
+            h[1][z].y -= syz * mz.x;
+            h[2][z].x += sxz * mx.y + syz * my.y;
+            h[2][z].y -= sxz * mx.x + syz * my.x;
+          }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int z = 0; z < NZ; ++z) col[(c * NZ + z) * K::LP] = h[c][z];
+  }
+}
+
+template <int L2, class K>
+__device__ __forceinline__ void yz_body(const DD& d, float2* __restrict__ A, const float2* __restrict__ Tz,
+                                        const float2* __restrict__ tw, int kx) {
+  using C = Line<L2>;
+  extern __shared__ float2 lds[];
+  const int g = threadIdx.x >> C::L2T, t = threadIdx.x & (C::T - 1);
+  const int nl = 3 * d.nz;
+  // lines li = c nz + z; thread groups past the last one take part in the
+  // barriers of lines of several wavefronts (in a spare buffer), or idle
+  float2 v[1][8];
+  for (int l0 = 0; l0 < nl; l0 += K::LB) {
+    const int li = l0 + g;
+    const bool in = li < nl;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[0][q] = make_float2(0.f, 0.f);
+    if (in) {
+      const float2* src = A + ((size_t)li * d.Hx + kx) * d.ny;
+#pragma unroll
+      for (int q = 0; q < C::EH; ++q) {
+        const int y = t + C::T * q;
+        if (y < d.ny) v[0][q] = src[y];
+      }
+    }
+    if (C::T > 64 || in) {
+      float2* line = lds + (in ? li : nl) * K::LP;
+      line_fft<L2, false, 1>(v, t, line, 0, tw);
+      if (in)
+#pragma unroll
+        for (int q = 0; q < C::E; ++q) line[iopad<L2>(t + C::T * q)] = v[0][q];
+    }
+  }
+  __syncthreads();
+  switch (d.nz) {
+    case 2: yz_convolve<2, L2, K>(d, lds, Tz, kx); break;
+    case 3: yz_convolve<3, L2, K>(d, lds, Tz, kx); break;
+    case 4: yz_convolve<4, L2, K>(d, lds, Tz, kx); break;
+    case 5: yz_convolve<5, L2, K>(d, lds, Tz, kx); break;
+    case 6: yz_convolve<6, L2, K>(d, lds, Tz, kx); break;
+    case 7: yz_convolve<7, L2, K>(d, lds, Tz, kx); break;
+    default: yz_convolve<8, L2, K>(d, lds, Tz, kx); break;
+  }
+  __syncthreads();
+  for (int l0 = 0; l0 < nl; l0 += K::LB) {
+    const int li = l0 + g;
+    const bool in = li < nl;
+    if (C::T > 64 || in) {
+      float2* line = lds + (in ? li : nl) * K::LP;
+      if (in)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[0][q] = q < C::E ? line[iopad<L2>(t + C::T * q)] : make_float2(0.f, 0.f);
+      line_sync<C::T>();
+      line_fft<L2, true, 1>(v, t, line, 0, tw);
+      if (in) {
+        float2* dst = A + ((size_t)li * d.Hx + kx) * d.ny;
+#pragma unroll
+        for (int q = 0; q < C::EH; ++q) {
+          const int y = t + C::T * q;
+          if (y < d.ny) dst[y] = v[0][q];
+        }
+      }
+    }
+  }
+}
+
+template <int L2, int TH>
+__global__ void __launch_bounds__((YzCfg<L2, TH>::THREADS))
+    k_yz(DD d, float2* __restrict__ A, const float2* __restrict__ Tz, const float2* __restrict__ tw) {
+  yz_body<L2, YzCfg<L2, TH>>(d, A, Tz, tw, blockIdx.x);
+}
+
+// Tz from the FP64 (x, y) sums in[((c nz + z) Hy + ky) Hx + kx].
+__global__ void k_few_table(const double* __restrict__ in, float2* __restrict__ Tz, int Hx, int Hy, int nz,
+                            double pref) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= Hx * Hy * nz) return;
+  const int ky = e % Hy, r = e / Hy, dz = r % nz, kx = r / nz;
+  float v[6];
+  for (int c = 0; c < 6; ++c) {
+    // xy: (-i)^2 of its two odd axes
+    const double sign = c == 3 ? -1.0 : 1.0;
+    v[c] = (float)(sign * pref * in[(((size_t)c * nz + dz) * Hy + ky) * Hx + kx]);
+  }
+  float2* out = Tz + ((size_t)kx * nz + dz) * 3 * Hy + ky;
+  out[0] = make_float2(v[0], v[1]);
+  out[Hy] = make_float2(v[2], v[3]);
+  out[2 * Hy] = make_float2(v[4], v[5]);
+}
+
 // ---------------------------------------------------------------- direct sum (small grids)
 
 __device__ __forceinline__ void direct_body(const DirectDesc& D, const DirectSource& S, float* __restrict__ h,
@@ -1052,6 +1222,28 @@ struct RunYpass2d {
   }
 };
 
+// Threads of the yz pass: enough groups for its 3 Nz lines, up to 1024.
+template <int L2>
+struct RunYz {
+  static void run(const DD& d, float2* A, const float2* Tz, const float2* tw, hipStream_t s) {
+    const int want = 3 * d.nz * Line<L2>::T;
+    if (want > 512) go<1024>(d, A, Tz, tw, s);
+    else if (want > 256) go<512>(d, A, Tz, tw, s);
+    else go<256>(d, A, Tz, tw, s);
+    checkLaunch("k_yz");
+  }
+  template <int TH>
+  static void go(const DD& d, float2* A, const float2* Tz, const float2* tw, hipStream_t s) {
+    using K = YzCfg<L2, TH>;
+    k_yz<L2, TH><<<d.Hx, K::THREADS, K::shm(d.nz), s>>>(d, A, Tz, tw);
+  }
+};
+
+template <int L2>
+struct YzShm {
+  static void run(int nz, size_t* shm) { *shm = YzCfg<L2, 256>::shm(nz); }
+};
+
 template <int L2>
 struct RunXinv {
   static void run(const DD& d, const float2* A, const uint8_t* geom, float* h, const float2* tw, hipStream_t s) {
@@ -1066,7 +1258,7 @@ struct RunXinv {
 // every size; a block finds its magnet through b2s and runs that magnet's
 // line length.
 // Block b of batched pass PASS (0 xfwd, 1 yfwd, 2 zpass, 3 yinv, 4 ypass2d,
-// 5 xinv): the member b2s[b] at its own line length.  X: packed state (pass
+// 5 xinv, 6 yz): the member b2s[b] at its own line length.  X: packed state (pass
 // 0), H: packed field (pass 5).
 // Lines of up to 2^PERSIST_MAXL2 points in the persistent step kernel (its
 // register budget is that of its largest body).
@@ -1111,6 +1303,10 @@ __device__ __forceinline__ void batch_pass_block(const BSeg* __restrict__ segs, 
 #define MPA_CALL(L) ypass2d_body<L, PointCfgB<L>>(s.d, s.A, s.T, s.tw[1], lb)
     MPA_L2_CASES(s.d.l2y, MPA_CALL)
 #undef MPA_CALL
+  } else if constexpr (PASS == 6) {
+#define MPA_CALL(L) yz_body<L, YzCfg<L, 256>>(s.d, s.A, s.Tz, s.tw[1], lb)
+    MPA_L2_CASES(s.d.l2y, MPA_CALL)
+#undef MPA_CALL
   } else {
 #define MPA_CALL(L) xinv_body<L, XinvCfgB<L>>(s.d, s.A, s.geom, H + s.off, s.tw[0], lb)
     MPA_L2_CASES(s.d.l2x, MPA_CALL)
@@ -1143,6 +1339,10 @@ __global__ void __launch_bounds__(256) k_ypass2d_b(const BSeg* __restrict__ segs
 __global__ void __launch_bounds__(256) k_xinv_b(const BSeg* __restrict__ segs, const int* __restrict__ b2s,
                                                 float* __restrict__ H) {
   batch_pass_block<5>(segs, b2s, xcd_remap(blockIdx.x, gridDim.x), nullptr, H);
+}
+
+__global__ void __launch_bounds__(256) k_yz_b(const BSeg* __restrict__ segs, const int* __restrict__ b2s) {
+  batch_pass_block<6>(segs, b2s, xcd_remap(blockIdx.x, gridDim.x), nullptr, nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -1250,6 +1450,7 @@ __device__ __forceinline__ void persist_demag(const bk::PhasePass& P, int b, con
     case 2: persist_pass<2>(segs, P.b2s, b, X, H); break;
     case 3: persist_pass<3>(segs, P.b2s, b, X, H); break;
     case 4: persist_pass<4>(segs, P.b2s, b, X, H); break;
+    case 6: persist_pass<6>(segs, P.b2s, b, X, H); break;
     default: persist_pass<5>(segs, P.b2s, b, X, H); break;
   }
 }
@@ -1343,6 +1544,10 @@ struct BatchShape {
         *blocks = grid_for(d.Hx, PointCfgB<L2>::PT);
         *shm = PointCfgB<L2>::SHM;
         break;
+      case 6:
+        *blocks = (unsigned)d.Hx;
+        *shm = YzCfg<L2, 256>::shm(d.nz);
+        break;
       default:
         *blocks = grid_for((d.nlines + 1) / 2, XinvCfgB<L2>::PB);
         *shm = XinvCfgB<L2>::SHM;
@@ -1359,6 +1564,7 @@ void run_batch_pass(int pass, unsigned nb, size_t shm, const BSeg* segs, const i
     case 2: k_zpass_b<<<nb, 256, shm, s>>>(segs, b2s); break;
     case 3: k_yinv_b<<<nb, 256, shm, s>>>(segs, b2s); break;
     case 4: k_ypass2d_b<<<nb, 256, shm, s>>>(segs, b2s); break;
+    case 6: k_yz_b<<<nb, 256, shm, s>>>(segs, b2s); break;
     default: k_xinv_b<<<nb, 256, shm, s>>>(segs, b2s, H); break;
   }
   checkLaunch("batched demag pass");
@@ -1404,6 +1610,12 @@ DemagPlan::DemagPlan(const DemagGeometry& g) : g_(g) {
   Hy_ = K_[1] / 2 + 1;
   Hz_ = K_[2] / 2 + 1;
   for (int a = 0; a < 3; ++a) make_twiddles(tw_[a], log2K_[a]);
+  if (g.n[2] >= 2 && g.n[2] <= FEW_MAX) {
+    // the y-lines of a kx in LDS
+    size_t shm = 0;
+    with_line<YzShm>(log2K_[1], g.n[2], &shm);
+    few_ = shm <= LDS_LIMIT - 1024;
+  }
   build_kernel(nullptr);
 }
 
@@ -1463,6 +1675,12 @@ void DemagPlan::build_kernel(hipStream_t s) {
                                                                         oddy, ct[1].get(), st[1].get());
   checkLaunch("k_trig_axis y");
   t1.release();
+  if (few_) {
+    Tz_.allocate((size_t)3 * Hx_ * Hy_ * nz);
+    k_few_table<<<grid_for((long long)Hx_ * Hy_ * nz), BLOCK, 0, s>>>(t2.get(), Tz_.get(), Hx_, Hy_, nz,
+                                                                      -MU0 / ((double)K_[0] * K_[1]));
+    checkLaunch("k_few_table");
+  }
   DeviceArray<double> t3((size_t)6 * Hz_ * Hy_ * Hx_);
   k_trig_axis<<<grid_for((long long)6 * Hz_ * Hy_ * Hx_), BLOCK, 0, s>>>(t2.get(), t3.get(), 1, nz, Hy_ * Hx_, K_[2],
                                                                         Hz_, oddz, ct[2].get(), st[2].get());
@@ -1485,7 +1703,7 @@ size_t DemagPlan::workspace_bytes() const {
 
 void DemagPlan::ensure_workspace() {
   if (A_.n == 0) A_.allocate(a_count());
-  if (!is2d() && B_.n == 0) B_.allocate(b_count());
+  if (!is2d() && !few_ && B_.n == 0) B_.allocate(b_count());
 }
 
 void DemagPlan::exec(const float* m, PS msat, const uint8_t* geom, float* h, hipStream_t s, Profiler* prof,
@@ -1577,6 +1795,9 @@ void DemagPlan::run(float2* A, float2* B, const float* m, PS msat, const uint8_t
   if (is2d()) {
     Timed t(prof, "k_ypass2d", pass_bytes(1), s);
     with_line<RunYpass2d>(d.l2y, d, A, T_.get(), tw_[1].get(), s);
+  } else if (few_) {
+    Timed t(prof, "k_yz", pass_bytes(1), s);
+    with_line<RunYz>(d.l2y, d, A, Tz_.get(), tw_[1].get(), s);
   } else {
     {
       Timed t(prof, "k_yfwd", pass_bytes(1), s);
@@ -1612,21 +1833,21 @@ DemagBatch::DemagBatch(const std::vector<Member>& members, long long cs) {
   }
   // pass -> (applies to a member, line length of its axis, plan pass index)
   auto applies = [&](int pass, int j) {
-    const bool flat = members[j].plan->is2d();
-    return pass == 0 || pass == 5 || (pass == 4 ? flat : !flat);
+    const bool flat = members[j].plan->is2d(), few = members[j].plan->few();
+    return pass == 0 || pass == 5 || (pass == 4 ? flat : (pass == 6 ? few : !flat && !few));
   };
   auto l2_of = [&](int pass, int j) {
     const DD& d = dd[j];
     return (pass == 0 || pass == 5) ? d.l2x : (pass == 2 ? d.l2z : d.l2y);
   };
   auto plan_pass = [&](int pass, int j) {
-    if (members[j].plan->is2d()) return pass == 0 ? 0 : (pass == 4 ? 1 : 2);
+    if (members[j].plan->npasses() == 3) return pass == 0 ? 0 : (pass == 5 ? 2 : 1);
     return pass == 5 ? 4 : pass;
   };
   // two independent chains: the members with a z transform (group 0) and the
   // single layers (group 1)
   for (int group = 0; group < 2; ++group)
-  for (int pass = 0; pass < 6; ++pass) {
+  for (int pass : {0, 1, 2, 3, 4, 6, 5}) {
     {
       std::vector<BSeg> segs;
       std::vector<int> b2s;
@@ -1649,6 +1870,7 @@ DemagBatch::DemagBatch(const std::vector<Member>& members, long long cs) {
         sg.B = p.B_.get();
         sg.T = p.T_.get();
         for (int a = 0; a < 3; ++a) sg.tw[a] = p.tw_[a].get();
+        sg.Tz = p.Tz_.get();
         sg.first = (int)b2s.size();
         b2s.insert(b2s.end(), nb, (int)segs.size());
         segs.push_back(sg);
@@ -1672,7 +1894,8 @@ DemagBatch::DemagBatch(const std::vector<Member>& members, long long cs) {
 
 void DemagBatch::exec(const float* X, float* H, hipStream_t s, Profiler* prof, hipStream_t s2, hipEvent_t fork,
                       hipEvent_t join) const {
-  static const char* names[] = {"k_xfwd_b", "k_yfwd_b", "k_zpass_b", "k_yinv_b", "k_ypass2d_b", "k_xinv_b"};
+  static const char* names[] = {"k_xfwd_b", "k_yfwd_b", "k_zpass_b", "k_yinv_b", "k_ypass2d_b", "k_xinv_b",
+                                "k_yz_b"};
   bool has[2] = {false, false};
   for (const Launch& L : launches_) has[L.group] = true;
   const bool split = s2 && fork && join && has[0] && has[1];
@@ -1713,7 +1936,8 @@ void batch_persist_launch(const bk::PersistArgs* a, int nsteps, unsigned gen0, i
 }
 
 void DemagBatch::exec_group(const float* X, float* H, int group, hipStream_t s, Profiler* prof) const {
-  static const char* names[] = {"k_xfwd_b", "k_yfwd_b", "k_zpass_b", "k_yinv_b", "k_ypass2d_b", "k_xinv_b"};
+  static const char* names[] = {"k_xfwd_b", "k_yfwd_b", "k_zpass_b", "k_yinv_b", "k_ypass2d_b", "k_xinv_b",
+                                "k_yz_b"};
   for (const Launch& L : launches_) {
     if (L.group != group) continue;
     Timed t(prof, names[L.pass], L.bytes, s);
@@ -1736,7 +1960,8 @@ double DemagBatch::algorithmic_bytes() const {
 const char* DemagPlan::pass_name(int i) const {
   static const char* n3[] = {"k_xfwd", "k_yfwd", "k_zpass", "k_yinv", "k_xinv"};
   static const char* n2[] = {"k_xfwd", "k_ypass2d", "k_xinv"};
-  return is2d() ? n2[i] : n3[i];
+  static const char* nf[] = {"k_xfwd", "k_yz", "k_xinv"};
+  return is2d() ? n2[i] : (few_ ? nf[i] : n3[i]);
 }
 
 double DemagPlan::pass_bytes(int i) const {
@@ -1747,6 +1972,10 @@ double DemagPlan::pass_bytes(int i) const {
   if (is2d()) {
     const double t = 16.0 * Hx_ * Hy_;  // xx, yy, zz, xy (xz = yz = 0 in a single layer)
     const double v[3] = {12 * N + xa, 2 * xa + t, xa + 12 * N};
+    return v[i];
+  }
+  if (few_) {
+    const double v[3] = {12 * N + xa, 2 * xa + 24.0 * Hx_ * Hy_ * nz, xa + 12 * N};
     return v[i];
   }
   const double t = 24.0 * Hx_ * Hy_ * Hz_;

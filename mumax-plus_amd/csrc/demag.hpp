@@ -49,17 +49,20 @@ class DemagPlan {
   void exec_noalloc(const float* m, PS msat, const uint8_t* geom, float* h, hipStream_t s);
   static size_t scratch_capacity();
   // Device bytes of the intermediates A (3 Nz Hx Ny complex) and, for a 3-D
-  // grid, B (3 Hx Ky Nz complex), each 256-byte aligned.
+  // grid, B (3 Hx Ky Nz complex; few layers need none of it), each 256-byte
+  // aligned.
   size_t workspace_bytes() const;
   // Allocates A and B if the plan does not hold them yet.
   void ensure_workspace();
+  // Whether y, z and the kernel are one pass (two to eight layers).
+  bool few() const { return few_; }
   // Whether exec sums the real-space kernel directly (small grids; one
   // launch, no intermediates), and the description of that sum.
   bool direct() const { return direct_; }
   const DirectDesc& direct_desc() const { return direct_desc_; }
   double direct_bytes() const;  // algorithmic HBM bytes of the direct sum
   // Pass names and algorithmic HBM bytes per pass.
-  int npasses() const { return is2d() ? 3 : 5; }
+  int npasses() const { return is2d() || few_ ? 3 : 5; }
   const char* pass_name(int i) const;
   double pass_bytes(int i) const;
 
@@ -94,6 +97,8 @@ class DemagPlan {
   DeviceArray<float2> A_, B_;
   DeviceArray<float> T_;
   DeviceArray<float2> tw_[3];
+  bool few_ = false;
+  DeviceArray<float2> Tz_;
   bool direct_ = false;
   DirectDesc direct_desc_{};
   DeviceArray<float4> direct_k4_;
@@ -130,7 +135,7 @@ class DemagBatch {
   // The launches' block tables, in launch order (each group's passes in
   // pass order), for the persistent step kernel.
   struct PassTable {
-    int pass;   // 0 xfwd, 1 yfwd, 2 zpass, 3 yinv, 4 ypass2d, 5 xinv
+    int pass;   // 0 xfwd, 1 yfwd, 2 zpass, 3 yinv, 4 ypass2d, 5 xinv, 6 yz
     int group;  // 0: members with a z transform, 1: single layers
     unsigned nblocks;
     size_t shm;
@@ -141,7 +146,7 @@ class DemagBatch {
 
  private:
   struct Launch {
-    int pass;   // 0 xfwd, 1 yfwd, 2 zpass, 3 yinv, 4 ypass2d, 5 xinv
+    int pass;   // 0 xfwd, 1 yfwd, 2 zpass, 3 yinv, 4 ypass2d, 5 xinv, 6 yz
     int group;  // 0: members with a z transform, 1: single layers
     size_t shm;
     unsigned nblocks;
