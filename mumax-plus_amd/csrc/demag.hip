@@ -871,26 +871,44 @@ __global__ void __launch_bounds__(XinvCfg<L2>::THREADS)
 // ky lie side by side, so a wavefront's loads are whole lines.
 constexpr int FEW_MAX = 8;
 
-template <int L2, int TH>
+// Shape of the pass for a magnet of nz layers in blocks of up to TH threads.
+// A batch (PACK) puts kpb consecutive kx into a block where the 3 Nz lines of
+// one do not fill it, so that few threads idle; a magnet's own launch takes one
+// kx per block, since it is the blocks that are few (64x64x2: 12.6 against 13.6
+// us packed).  lb lines are transformed at a time, with just the threads that
+// they need (512x512x2: 53.3 us with 768, 56.7 with 1024), but as many as fit
+// in 1024 where it takes several rounds (the column sums want the wavefronts:
+// 300x220x6 56.9 against 61.3 us with 576).
+template <int L2, int TH, bool PACK = false>
 struct YzCfg {
   using C = Line<L2>;
-  static constexpr int LB = TH / C::T;  // lines transformed at a time
-  static constexpr int THREADS = LB * C::T;
+  static constexpr bool packs = PACK;
   // transforms and the column reads take consecutive elements of a line
   static constexpr int LP = C::stride(C::fft_target());
+  __host__ __device__ static int kpb(int nz) {
+    const int k = PACK ? TH / (3 * nz * C::T) : 1;
+    return k > 1 ? k : 1;
+  }
+  __host__ __device__ static int lb(int nz) {
+    const int nl = 3 * nz * kpb(nz), rounds = (nl * C::T + TH - 1) / TH;
+    return TH >= 1024 && rounds > 1 ? TH / C::T : (nl + rounds - 1) / rounds;
+  }
+  __host__ __device__ static int threads(int nz) { return (lb(nz) * C::T + 63) / 64 * 64; }
   // lines of several wavefronts: one more buffer for the groups past the last line
-  static size_t shm(int nz) { return (size_t)(3 * nz + (C::T > 64 ? 1 : 0)) * LP * sizeof(float2); }
+  static size_t shm(int nz) { return (size_t)(3 * nz * kpb(nz) + (C::T > 64 ? 1 : 0)) * LP * sizeof(float2); }
 };
 
 template <int NZ, int L2, class K>
-__device__ __forceinline__ void yz_convolve(const DD& d, float2* lds, const float2* __restrict__ Tz, int kx) {
+__device__ __forceinline__ void yz_convolve(const DD& d, float2* lds, const float2* __restrict__ Tz, int kx0,
+                                            int nkx) {
   using C = Line<L2>;
-  const float2* row = Tz + (size_t)kx * NZ * 3 * d.Hy;
-  for (int ky = threadIdx.x; ky < C::L; ky += K::THREADS) {
+  for (int e = threadIdx.x; e < (K::packs ? nkx : 1) * C::L; e += blockDim.x) {
+    const int kxl = K::packs ? e >> L2 : 0, ky = e & (C::L - 1);
+    const float2* row = Tz + (size_t)(kx0 + kxl) * NZ * 3 * d.Hy;
     const bool up = ky > (C::L >> 1);  // mirrored: the components odd in y change sign
     const int kh = up ? C::L - ky : ky;
     const float sy = up ? -1.f : 1.f;
-    float2* col = lds + iopad<L2>(ky);
+    float2* col = lds + kxl * 3 * NZ * K::LP + iopad<L2>(ky);
     float2 m[3][NZ], h[3][NZ];
 #pragma unroll
     for (int c = 0; c < 3; ++c)
@@ -936,23 +954,29 @@ __device__ __forceinline__ void yz_convolve(const DD& d, float2* lds, const floa
   }
 }
 
-template <int L2, class K>
+template <int L2, class K, int NZMAX>
 __device__ __forceinline__ void yz_body(const DD& d, float2* __restrict__ A, const float2* __restrict__ Tz,
-                                        const float2* __restrict__ tw, int kx) {
+                                        const float2* __restrict__ tw, int blk) {
   using C = Line<L2>;
   extern __shared__ float2 lds[];
   const int g = threadIdx.x >> C::L2T, t = threadIdx.x & (C::T - 1);
-  const int nl = 3 * d.nz;
-  // lines li = c nz + z; thread groups past the last one take part in the
-  // barriers of lines of several wavefronts (in a spare buffer), or idle
+  const int kpb = K::kpb(d.nz), kx0 = blk * kpb, nkx = min(kpb, d.Hx - kx0);
+  const int n3 = 3 * d.nz, nl = n3 * nkx, lb = K::lb(d.nz);
+  // start of line li = (kxl, c, z) in A; thread groups past the last line take
+  // part in the barriers of lines of several wavefronts (in a spare buffer),
+  // or idle
+  auto aline = [&](int li) {
+    const int kxl = K::packs ? li / n3 : 0;
+    return ((size_t)(li - kxl * n3) * d.Hx + kx0 + kxl) * d.ny;
+  };
   float2 v[1][8];
-  for (int l0 = 0; l0 < nl; l0 += K::LB) {
+  for (int l0 = 0; l0 < nl; l0 += lb) {
     const int li = l0 + g;
-    const bool in = li < nl;
+    const bool in = g < lb && li < nl;
 #pragma unroll
     for (int q = 0; q < 8; ++q) v[0][q] = make_float2(0.f, 0.f);
     if (in) {
-      const float2* src = A + ((size_t)li * d.Hx + kx) * d.ny;
+      const float2* src = A + aline(li);
 #pragma unroll
       for (int q = 0; q < C::EH; ++q) {
         const int y = t + C::T * q;
@@ -969,18 +993,19 @@ __device__ __forceinline__ void yz_body(const DD& d, float2* __restrict__ A, con
   }
   __syncthreads();
   switch (d.nz) {
-    case 2: yz_convolve<2, L2, K>(d, lds, Tz, kx); break;
-    case 3: yz_convolve<3, L2, K>(d, lds, Tz, kx); break;
-    case 4: yz_convolve<4, L2, K>(d, lds, Tz, kx); break;
-    case 5: yz_convolve<5, L2, K>(d, lds, Tz, kx); break;
-    case 6: yz_convolve<6, L2, K>(d, lds, Tz, kx); break;
-    case 7: yz_convolve<7, L2, K>(d, lds, Tz, kx); break;
-    default: yz_convolve<8, L2, K>(d, lds, Tz, kx); break;
+    case 2: yz_convolve<2, L2, K>(d, lds, Tz, kx0, nkx); break;
+    case 3: yz_convolve<3, L2, K>(d, lds, Tz, kx0, nkx); break;
+    case 4: yz_convolve<4, L2, K>(d, lds, Tz, kx0, nkx); break;
+    case 5: if constexpr (NZMAX >= 5) yz_convolve<5, L2, K>(d, lds, Tz, kx0, nkx); break;
+    case 6: if constexpr (NZMAX >= 6) yz_convolve<6, L2, K>(d, lds, Tz, kx0, nkx); break;
+    case 7: if constexpr (NZMAX >= 7) yz_convolve<7, L2, K>(d, lds, Tz, kx0, nkx); break;
+    case 8: if constexpr (NZMAX >= 8) yz_convolve<8, L2, K>(d, lds, Tz, kx0, nkx); break;
+    default: break;
   }
   __syncthreads();
-  for (int l0 = 0; l0 < nl; l0 += K::LB) {
+  for (int l0 = 0; l0 < nl; l0 += lb) {
     const int li = l0 + g;
-    const bool in = li < nl;
+    const bool in = g < lb && li < nl;
     if (C::T > 64 || in) {
       float2* line = lds + (in ? li : nl) * K::LP;
       if (in)
@@ -989,7 +1014,7 @@ __device__ __forceinline__ void yz_body(const DD& d, float2* __restrict__ A, con
       line_sync<C::T>();
       line_fft<L2, true, 1>(v, t, line, 0, tw);
       if (in) {
-        float2* dst = A + ((size_t)li * d.Hx + kx) * d.ny;
+        float2* dst = A + aline(li);
 #pragma unroll
         for (int q = 0; q < C::EH; ++q) {
           const int y = t + C::T * q;
@@ -1000,10 +1025,12 @@ __device__ __forceinline__ void yz_body(const DD& d, float2* __restrict__ A, con
   }
 }
 
-template <int L2, int TH>
-__global__ void __launch_bounds__((YzCfg<L2, TH>::THREADS))
+// TH: the most threads of a block, NZMAX: the most layers (a block keeps 12
+// values per layer in registers, so few-layer grids get the leaner instance).
+template <int L2, int TH, int NZMAX>
+__global__ void __launch_bounds__(TH)
     k_yz(DD d, float2* __restrict__ A, const float2* __restrict__ Tz, const float2* __restrict__ tw) {
-  yz_body<L2, YzCfg<L2, TH>>(d, A, Tz, tw, blockIdx.x);
+  yz_body<L2, YzCfg<L2, TH>, NZMAX>(d, A, Tz, tw, xcd_remap(blockIdx.x, gridDim.x));
 }
 
 // Tz from the FP64 (x, y) sums in[((c nz + z) Hy + ky) Hx + kx].
@@ -1222,26 +1249,34 @@ struct RunYpass2d {
   }
 };
 
-// Threads of the yz pass: enough groups for its 3 Nz lines, up to 1024.
+// Blocks of up to 256 threads where the lines of a kx fit, of up to 640 (two
+// to three wavefronts per SIMD with 168 registers) or 1024 otherwise.
 template <int L2>
 struct RunYz {
   static void run(const DD& d, float2* A, const float2* Tz, const float2* tw, hipStream_t s) {
     const int want = 3 * d.nz * Line<L2>::T;
-    if (want > 512) go<1024>(d, A, Tz, tw, s);
-    else if (want > 256) go<512>(d, A, Tz, tw, s);
-    else go<256>(d, A, Tz, tw, s);
+    if (want <= 256) nz<256>(d, A, Tz, tw, s);
+    else if (want <= 640) nz<640>(d, A, Tz, tw, s);
+    else nz<1024>(d, A, Tz, tw, s);
     checkLaunch("k_yz");
   }
   template <int TH>
+  static void nz(const DD& d, float2* A, const float2* Tz, const float2* tw, hipStream_t s) {
+    if (d.nz <= 4) go<TH, 4>(d, A, Tz, tw, s);
+    else go<TH, 8>(d, A, Tz, tw, s);
+  }
+  template <int TH, int NZMAX>
   static void go(const DD& d, float2* A, const float2* Tz, const float2* tw, hipStream_t s) {
-    using K = YzCfg<L2, TH>;
-    k_yz<L2, TH><<<d.Hx, K::THREADS, K::shm(d.nz), s>>>(d, A, Tz, tw);
+    using Cfg = YzCfg<L2, TH>;
+    const unsigned blocks = grid_for(d.Hx, Cfg::kpb(d.nz)), threads = (unsigned)Cfg::threads(d.nz);
+    k_yz<L2, TH, NZMAX><<<blocks, threads, Cfg::shm(d.nz), s>>>(d, A, Tz, tw);
   }
 };
 
 template <int L2>
 struct YzShm {
-  static void run(int nz, size_t* shm) { *shm = YzCfg<L2, 256>::shm(nz); }
+  // the lines of one kx
+  static void run(int nz, size_t* shm) { *shm = (size_t)(3 * nz + 1) * YzCfg<L2, 256>::LP * sizeof(float2); }
 };
 
 template <int L2>
@@ -1264,7 +1299,7 @@ struct RunXinv {
 // register budget is that of its largest body).
 constexpr int PERSIST_MAXL2 = 8;
 
-template <int PASS, int LMAX = MAXL2>
+template <int PASS, int LMAX = MAXL2, int NZMAX = FEW_MAX>
 __device__ __forceinline__ void batch_pass_block(const BSeg* __restrict__ segs, const int* __restrict__ b2s, int b,
                                                  const float* __restrict__ X, float* __restrict__ H) {
   const BSeg s = segs[b2s[b]];
@@ -1304,7 +1339,7 @@ __device__ __forceinline__ void batch_pass_block(const BSeg* __restrict__ segs, 
     MPA_L2_CASES(s.d.l2y, MPA_CALL)
 #undef MPA_CALL
   } else if constexpr (PASS == 6) {
-#define MPA_CALL(L) yz_body<L, YzCfg<L, 256>>(s.d, s.A, s.Tz, s.tw[1], lb)
+#define MPA_CALL(L) yz_body<L, YzCfg<L, 256, true>, NZMAX>(s.d, s.A, s.Tz, s.tw[1], lb)
     MPA_L2_CASES(s.d.l2y, MPA_CALL)
 #undef MPA_CALL
   } else {
@@ -1341,8 +1376,9 @@ __global__ void __launch_bounds__(256) k_xinv_b(const BSeg* __restrict__ segs, c
   batch_pass_block<5>(segs, b2s, xcd_remap(blockIdx.x, gridDim.x), nullptr, H);
 }
 
+template <int LMAX, int NZMAX>
 __global__ void __launch_bounds__(256) k_yz_b(const BSeg* __restrict__ segs, const int* __restrict__ b2s) {
-  batch_pass_block<6>(segs, b2s, xcd_remap(blockIdx.x, gridDim.x), nullptr, nullptr);
+  batch_pass_block<6, LMAX, NZMAX>(segs, b2s, xcd_remap(blockIdx.x, gridDim.x), nullptr, nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -1545,8 +1581,8 @@ struct BatchShape {
         *shm = PointCfgB<L2>::SHM;
         break;
       case 6:
-        *blocks = (unsigned)d.Hx;
-        *shm = YzCfg<L2, 256>::shm(d.nz);
+        *blocks = grid_for(d.Hx, YzCfg<L2, 256, true>::kpb(d.nz));
+        *shm = YzCfg<L2, 256, true>::shm(d.nz);
         break;
       default:
         *blocks = grid_for((d.nlines + 1) / 2, XinvCfgB<L2>::PB);
@@ -1556,7 +1592,7 @@ struct BatchShape {
   }
 };
 
-void run_batch_pass(int pass, unsigned nb, size_t shm, const BSeg* segs, const int* b2s, const float* X, float* H,
+void run_batch_pass(int pass, bool lean, unsigned nb, size_t shm, const BSeg* segs, const int* b2s, const float* X, float* H,
                     hipStream_t s) {
   switch (pass) {
     case 0: k_xfwd_b<<<nb, 256, shm, s>>>(segs, b2s, X); break;
@@ -1564,7 +1600,11 @@ void run_batch_pass(int pass, unsigned nb, size_t shm, const BSeg* segs, const i
     case 2: k_zpass_b<<<nb, 256, shm, s>>>(segs, b2s); break;
     case 3: k_yinv_b<<<nb, 256, shm, s>>>(segs, b2s); break;
     case 4: k_ypass2d_b<<<nb, 256, shm, s>>>(segs, b2s); break;
-    case 6: k_yz_b<<<nb, 256, shm, s>>>(segs, b2s); break;
+    case 6:
+      // lines of 256 points and four layers at most: 2.4 times the wavefronts
+      if (lean) k_yz_b<8, 4><<<nb, 256, shm, s>>>(segs, b2s);
+      else k_yz_b<MAXL2, FEW_MAX><<<nb, 256, shm, s>>>(segs, b2s);
+      break;
     default: k_xinv_b<<<nb, 256, shm, s>>>(segs, b2s, H); break;
   }
   checkLaunch("batched demag pass");
@@ -1853,12 +1893,14 @@ DemagBatch::DemagBatch(const std::vector<Member>& members, long long cs) {
       std::vector<int> b2s;
       double bytes = 0.0;
       size_t shm_max = 0;
+      bool lean = true;
       for (int j = 0; j < M; ++j) {
         if ((members[j].plan->is2d() ? 1 : 0) != group || !applies(pass, j)) continue;
         unsigned nb = 0;
         size_t shm = 0;
         with_line<BatchShape>(l2_of(pass, j), pass, dd[j], &nb, &shm);
         shm_max = shm > shm_max ? shm : shm_max;
+        lean = lean && dd[j].l2y <= 8 && dd[j].nz <= 4;
         members[j].plan->ensure_workspace();
         const DemagPlan& p = *members[j].plan;
         BSeg sg{};
@@ -1881,6 +1923,7 @@ DemagBatch::DemagBatch(const std::vector<Member>& members, long long cs) {
       L.pass = pass;
       L.group = group;
       L.shm = shm_max;
+      L.lean = lean;
       L.nblocks = (unsigned)b2s.size();
       L.bytes = bytes;
       L.segs.allocate(segs.size() * sizeof(BSeg));
@@ -1907,7 +1950,7 @@ void DemagBatch::exec(const float* X, float* H, hipStream_t s, Profiler* prof, h
   for (const Launch& L : launches_) {
     hipStream_t st = split && L.group == 1 ? s2 : s;
     Timed t(prof, names[L.pass], L.bytes, st);
-    run_batch_pass(L.pass, L.nblocks, L.shm, reinterpret_cast<const BSeg*>(L.segs.get()), L.b2s.get(), X, H, st);
+    run_batch_pass(L.pass, L.lean, L.nblocks, L.shm, reinterpret_cast<const BSeg*>(L.segs.get()), L.b2s.get(), X, H, st);
   }
   if (split) {
     HIP_CHECK(hipEventRecord(join, s2));
@@ -1941,7 +1984,7 @@ void DemagBatch::exec_group(const float* X, float* H, int group, hipStream_t s, 
   for (const Launch& L : launches_) {
     if (L.group != group) continue;
     Timed t(prof, names[L.pass], L.bytes, s);
-    run_batch_pass(L.pass, L.nblocks, L.shm, reinterpret_cast<const BSeg*>(L.segs.get()), L.b2s.get(), X, H, s);
+    run_batch_pass(L.pass, L.lean, L.nblocks, L.shm, reinterpret_cast<const BSeg*>(L.segs.get()), L.b2s.get(), X, H, s);
   }
 }
 

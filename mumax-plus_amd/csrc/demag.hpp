@@ -148,6 +148,7 @@ class DemagBatch {
   struct Launch {
     int pass;   // 0 xfwd, 1 yfwd, 2 zpass, 3 yinv, 4 ypass2d, 5 xinv, 6 yz
     int group;  // 0: members with a z transform, 1: single layers
+    bool lean;  // lines of up to 256 points, up to four layers
     size_t shm;
     unsigned nblocks;
     DeviceArray<char> segs;
