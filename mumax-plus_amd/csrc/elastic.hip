@@ -11,23 +11,24 @@ constexpr int BLOCK = 256;
 
 using namespace elc;
 
+template <bool FILM>
 __global__ void __launch_bounds__(BLOCK) k_strain(ElDesc d, const float* __restrict__ u, float* __restrict__ strain,
                                                   float* __restrict__ stress) {
   const int idx = xcd_remap(blockIdx.x, gridDim.x) * BLOCK + threadIdx.x;
   const int N = d.ncell;
   if (idx >= N) return;
-  if (!in_geo(d, idx)) {
+  if (!FILM && !in_geo(d, idx)) {
     for (int c = 0; c < 6; ++c) {
       strain[(size_t)c * N + idx] = 0.f;
       if (stress) stress[(size_t)c * N + idx] = 0.f;
     }
     return;
   }
-  const int x = idx % d.nx, y = (idx / d.nx) % d.ny, z = idx / (d.nx * d.ny);
+  const int x = idx % d.nx, y = FILM ? idx / d.nx : (idx / d.nx) % d.ny, z = FILM ? 0 : idx / (d.nx * d.ny);
   const float3 u0 = ld3(u, idx, N);
-  const float3 dx = deriv(d, u, axis_nb(d, x, y, z, 0), 0, u0);  // d_x u
-  const float3 dy = deriv(d, u, axis_nb(d, x, y, z, 1), 1, u0);
-  const float3 dz = deriv(d, u, axis_nb(d, x, y, z, 2), 2, u0);
+  const float3 dx = deriv(d, u, axis_nb<FILM>(d, x, y, z, 0), 0, u0);  // d_x u
+  const float3 dy = deriv(d, u, axis_nb<FILM>(d, x, y, z, 1), 1, u0);
+  const float3 dz = deriv(d, u, axis_nb<FILM>(d, x, y, z, 2), 2, u0);
   // straintensor.cu:81-97: e_ii = d_i u_i, e_ij = (d_i u_j + d_j u_i)/2
   const float e[6] = {dx.x, dy.y, dz.z, 0.5f * (dx.y + dy.x), 0.5f * (dx.z + dz.x), 0.5f * (dy.z + dz.y)};
   for (int c = 0; c < 6; ++c) strain[(size_t)c * N + idx] = e[c];
@@ -41,26 +42,27 @@ __global__ void __launch_bounds__(BLOCK) k_strain(ElDesc d, const float* __restr
   }
 }
 
+template <bool FILM>
 __global__ void __launch_bounds__(BLOCK) k_elastic(ElDesc d, const float* __restrict__ stress,
                                                    const float* __restrict__ v, MEForce a, MEForce b,
                                                    float* __restrict__ out, int mode) {
   const int idx = xcd_remap(blockIdx.x, gridDim.x) * BLOCK + threadIdx.x;
   if (idx >= d.ncell) return;
-  elastic_cell(d, stress, v, a, b, out, mode, idx);
+  elastic_cell<FILM>(d, stress, v, a, b, out, mode, idx);
 }
 
-template <int NK>
+template <int NK, bool FILM>
 __global__ void __launch_bounds__(BLOCK) k_elastic_next(ElDesc d, const float* __restrict__ stress,
                                                         const float* __restrict__ v, MEForce a, MEForce b,
                                                         float* __restrict__ out, ElNext nx) {
   const int idx = xcd_remap(blockIdx.x, gridDim.x) * BLOCK + threadIdx.x;
   const int N = d.ncell;
   if (idx >= N) return;
-  const float3 f = elastic_term(d, stress, v, a, b, EL_ACCEL, idx);
+  const float3 f = elastic_term<FILM>(d, stress, v, a, b, EL_ACCEL, idx);
   out[idx] = f.x;
   out[(size_t)N + idx] = f.y;
   out[(size_t)2 * N + idx] = f.z;
-  elastic_next<NK>(d, nx, f, idx);
+  elastic_next<NK, FILM>(d, nx, f, idx);
 }
 
 __global__ void __launch_bounds__(BLOCK) k_elastic_local(ElDesc d, const float* __restrict__ stress,
@@ -92,12 +94,24 @@ __global__ void __launch_bounds__(BLOCK) k_elastic_local(ElDesc d, const float* 
   }
 }
 
+// A single layer that is periodic over exactly its own extent in x and y, and
+// not in z, without a mask: the stencils are the five-point ones everywhere and
+// nothing varies along z, so neighbour tables, boundary rules and the z axis
+// drop out at compile time (elastic_cell.hpp, FILM).  The same formulas.  512 x
+// 512: strain 8.6 -> 5.4 us, acceleration with the next stage 13.3-17.3 ->
+// 9.5-13.0 us.
+bool elastic_film(const ElDesc& d) {
+  return !d.geom && d.nz == 1 && d.mgz == 0 && d.mgx == d.nx && d.mgy == d.ny && d.mox == d.ox && d.moy == d.oy &&
+         d.nx >= 3 && d.ny >= 3;
+}
+
 unsigned blocks(int n) { return (unsigned)((n + BLOCK - 1) / BLOCK); }
 
 }  // namespace
 
 void launch_strain(const ElDesc& d, const float* u, float* strain, float* stress, hipStream_t s) {
-  k_strain<<<blocks(d.ncell), BLOCK, 0, s>>>(d, u, strain, stress);
+  if (elastic_film(d)) k_strain<true><<<blocks(d.ncell), BLOCK, 0, s>>>(d, u, strain, stress);
+  else k_strain<false><<<blocks(d.ncell), BLOCK, 0, s>>>(d, u, strain, stress);
   checkLaunch("k_strain");
 }
 
@@ -105,7 +119,8 @@ void launch_elastic(const ElDesc& d, const float* stress, const float* v, const 
                     float* out, ElMode mode, hipStream_t s) {
   if ((mode == EL_FORCE || ((mode == EL_BODY || mode == EL_ACCEL) && d.elastic)) && !stress)
     throw Error(MPA_ERR_RUNTIME, "elastic force needs the stress tensor");
-  k_elastic<<<blocks(d.ncell), BLOCK, 0, s>>>(d, stress, v, a, b, out, (int)mode);
+  if (elastic_film(d)) k_elastic<true><<<blocks(d.ncell), BLOCK, 0, s>>>(d, stress, v, a, b, out, (int)mode);
+  else k_elastic<false><<<blocks(d.ncell), BLOCK, 0, s>>>(d, stress, v, a, b, out, (int)mode);
   checkLaunch("k_elastic");
 }
 
@@ -113,15 +128,20 @@ void launch_elastic_next(const ElDesc& d, const float* stress, const float* v, c
                          float* out, const ElNext& nx, hipStream_t s) {
   if (d.elastic && !stress) throw Error(MPA_ERR_RUNTIME, "elastic force needs the stress tensor");
   const unsigned g = blocks(d.ncell);
+  const bool film = elastic_film(d);
+#define MPA_EL_NEXT(K)                                                            \
+  if (film) k_elastic_next<K, true><<<g, BLOCK, 0, s>>>(d, stress, v, a, b, out, nx); \
+  else k_elastic_next<K, false><<<g, BLOCK, 0, s>>>(d, stress, v, a, b, out, nx);
   switch (nx.nk) {
-    case 0: k_elastic_next<0><<<g, BLOCK, 0, s>>>(d, stress, v, a, b, out, nx); break;
-    case 1: k_elastic_next<1><<<g, BLOCK, 0, s>>>(d, stress, v, a, b, out, nx); break;
-    case 2: k_elastic_next<2><<<g, BLOCK, 0, s>>>(d, stress, v, a, b, out, nx); break;
-    case 3: k_elastic_next<3><<<g, BLOCK, 0, s>>>(d, stress, v, a, b, out, nx); break;
-    case 4: k_elastic_next<4><<<g, BLOCK, 0, s>>>(d, stress, v, a, b, out, nx); break;
-    case 5: k_elastic_next<5><<<g, BLOCK, 0, s>>>(d, stress, v, a, b, out, nx); break;
+    case 0: MPA_EL_NEXT(0) break;
+    case 1: MPA_EL_NEXT(1) break;
+    case 2: MPA_EL_NEXT(2) break;
+    case 3: MPA_EL_NEXT(3) break;
+    case 4: MPA_EL_NEXT(4) break;
+    case 5: MPA_EL_NEXT(5) break;
     default: throw Error(MPA_ERR_RUNTIME, "launch_elastic_next: 0 to 5 earlier derivatives");
   }
+#undef MPA_EL_NEXT
   checkLaunch("k_elastic_next");
 }
 

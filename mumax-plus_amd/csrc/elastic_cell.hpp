@@ -41,9 +41,24 @@ struct AxisNb {
   bool g[4];
 };
 
+// FILM: a single layer without mask, periodic over its own extent in x and y
+// (elastic_film): every in-plane neighbour exists, one wrap away at most, and
+// there is none along z.
+template <bool FILM = false>
 __device__ __forceinline__ AxisNb axis_nb(const ElDesc& d, int x, int y, int z, int axis) {
   AxisNb a;
   const int k[4] = {-2, -1, 1, 2};
+  if constexpr (FILM) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int n = axis == 0 ? d.nx : d.ny, c = axis == 0 ? x : y;
+      int l = c + k[q];
+      l = l < 0 ? l + n : (l >= n ? l - n : l);
+      a.i[q] = axis == 2 ? 0 : (axis == 0 ? y * d.nx + l : l * d.nx + x);
+      a.g[q] = axis != 2;
+    }
+    return a;
+  }
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     a.i[q] = shifted(d, x, y, z, axis, k[q]);
@@ -125,16 +140,17 @@ __device__ __forceinline__ float3 me_force(const ElDesc& d, const MEForce& a, in
 }
 
 // The selected elastic term at cell idx (< ncell; see ElMode).
+template <bool FILM = false>
 __device__ __forceinline__ float3 elastic_term(const ElDesc& d, const float* __restrict__ stress,
                                                const float* __restrict__ v, const MEForce& a, const MEForce& b,
                                                int mode, int idx) {
   const int N = d.ncell;
   float3 f = f3(0.f, 0.f, 0.f);
-  if (in_geo(d, idx)) {
-    const int x = idx % d.nx, y = (idx / d.nx) % d.ny, z = idx / (d.nx * d.ny);
+  if (FILM || in_geo(d, idx)) {
+    const int x = idx % d.nx, y = FILM ? idx / d.nx : (idx / d.nx) % d.ny, z = FILM ? 0 : idx / (d.nx * d.ny);
     AxisNb nb[3];
 #pragma unroll
-    for (int ax = 0; ax < 3; ++ax) nb[ax] = axis_nb(d, x, y, z, ax);
+    for (int ax = 0; ax < 3; ++ax) nb[ax] = axis_nb<FILM>(d, x, y, z, ax);
     const bool body = mode == EL_BODY || mode == EL_ACCEL;
     if (mode == EL_FORCE || (body && d.elastic)) f = f + stress_divergence(d, stress, idx, nb);
     if (body && d.ext) f = f + d.fext.at(idx, N);
@@ -151,11 +167,12 @@ __device__ __forceinline__ float3 elastic_term(const ElDesc& d, const float* __r
 
 // The selected elastic term at cell idx (< ncell), written to out
 // (k_elastic's cell).
+template <bool FILM = false>
 __device__ __forceinline__ void elastic_cell(const ElDesc& d, const float* __restrict__ stress,
                                              const float* __restrict__ v, const MEForce& a, const MEForce& b,
                                              float* __restrict__ out, int mode, int idx) {
   const int N = d.ncell;
-  const float3 f = elastic_term(d, stress, v, a, b, mode, idx);
+  const float3 f = elastic_term<FILM>(d, stress, v, a, b, mode, idx);
   out[idx] = f.x;
   out[(size_t)N + idx] = f.y;
   out[(size_t)2 * N + idx] = f.z;
@@ -164,10 +181,10 @@ __device__ __forceinline__ void elastic_cell(const ElDesc& d, const float* __res
 // The next stage state of (u, v) at cell idx from the acceleration f just
 // computed there (ElNext); NK = nx.nk, known at compile time so that every
 // load is issued before the sums.
-template <int NK>
+template <int NK, bool FILM = false>
 __device__ __forceinline__ void elastic_next(const ElDesc& d, const ElNext& nx, float3 f, int idx) {
   const int N = d.ncell;
-  const bool in = in_geo(d, idx);
+  const bool in = FILM || in_geo(d, idx);
   const float fc[3] = {f.x, f.y, f.z};
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
