@@ -10,6 +10,8 @@
 // two-level FP64 sum.
 #include "rk.hpp"
 
+#include <chrono>
+
 namespace mpa {
 
 namespace {
@@ -187,21 +189,41 @@ __device__ __forceinline__ float block_max(float v) {
   return v;
 }
 
+// max over cells of |sum_j c_j k_j|.  NK >= 0: NK derivatives, a compile-time
+// count, so a thread's loads are in flight together (NK < 0: co.nk read at run
+// time).  The blocks merge their maxima into w.max; the last one to finish puts
+// the result, tagged with the call's number, into host memory, so that no copy
+// launch follows, and leaves w zeroed for the next call.
+template <int NK>
 __global__ void __launch_bounds__(BLOCK) k_combo_maxnorm(Combo co, int N, const uint8_t* __restrict__ geom,
-                                                         unsigned* __restrict__ result) {
+                                                         NormWords* __restrict__ w,
+                                                         unsigned long long* __restrict__ host, unsigned tag) {
   float best = 0.f;
   for (int idx = blockIdx.x * BLOCK + threadIdx.x; idx < N; idx += gridDim.x * BLOCK) {
     if (geom && !geom[idx]) continue;
     float e[3];
+#pragma unroll
     for (int c = 0; c < 3; ++c) {
       float a = 0.f;
-      for (int j = 0; j < co.nk; ++j) a += co.c[j] * co.k[j][(size_t)c * N + idx];
+#pragma unroll
+      for (int j = 0; j < (NK >= 0 ? NK : MAX_STAGES); ++j) {
+        if (NK < 0 && j >= co.nk) break;
+        a += co.c[j] * co.k[j][(size_t)c * N + idx];
+      }
       e[c] = a;
     }
     best = fmaxf(best, sqrtf(e[0] * e[0] + e[1] * e[1] + e[2] * e[2]));
   }
   best = block_max(best);
-  if (threadIdx.x == 0) atomicMax(result, __float_as_uint(best));
+  if (threadIdx.x == 0) {
+    atomicMax(&w->max, __float_as_uint(best));
+    __threadfence();
+    if (atomicAdd(&w->done, 1u) == gridDim.x - 1) {
+      const unsigned bits = atomicExch(&w->max, 0u);
+      atomicExch(&w->done, 0u);
+      __hip_atomic_store(host, ((unsigned long long)tag << 32) | bits, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
 }
 
 __global__ void k_zero_u32(unsigned* p) { *p = 0u; }
@@ -375,15 +397,44 @@ void launch_combine_batch(const CombineJob* jobs, int njobs, hipStream_t s) {
   checkLaunch("k_combine_batch");
 }
 
-Reducer::Reducer() : maxbits_(1), partials_((size_t)3 * SUM_BLOCKS + 3) {}
+Reducer::Reducer() : maxbits_(1), partials_((size_t)3 * SUM_BLOCKS + 3), words_(1) {
+  HIP_CHECK(hipMemset(words_.get(), 0, words_.bytes()));
+  HIP_CHECK(hipStreamSynchronize(nullptr));
+  HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_), sizeof(*host_), hipHostMallocDefault));
+  *host_ = 0;
+}
+
+Reducer::~Reducer() {
+  if (host_) (void)hipHostFree(host_);
+}
 
 float Reducer::max_combo_norm(const Combo& co, int N, const uint8_t* geom, hipStream_t s) {
-  k_zero_u32<<<1, 1, 0, s>>>(maxbits_.get());
-  k_combo_maxnorm<<<reduce_blocks(N), BLOCK, 0, s>>>(co, N, geom, maxbits_.get());
+  const unsigned tag = ++tag_ ? tag_ : ++tag_;  // 0 is the initial content
+  const int nb = reduce_blocks(N);
+  auto launch = [&](auto kernel) { kernel<<<nb, BLOCK, 0, s>>>(co, N, geom, words_.get(), host_, tag); };
+  switch (co.nk) {
+    case 1: launch(k_combo_maxnorm<1>); break;
+    case 4: launch(k_combo_maxnorm<4>); break;
+    case 5: launch(k_combo_maxnorm<5>); break;
+    case 6: launch(k_combo_maxnorm<6>); break;
+    default: launch(k_combo_maxnorm<-1>); break;
+  }
   checkLaunch("k_combo_maxnorm");
-  unsigned bits = 0;
-  HIP_CHECK(hipMemcpyAsync(&bits, maxbits_.get(), sizeof(unsigned), hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipStreamSynchronize(s));
+  // the result arrives a microsecond after the kernel's last block; waiting for
+  // the stream and copying a word would cost the step controller ten more
+  const auto start = std::chrono::steady_clock::now();
+  auto word = [&] { return __atomic_load_n(host_, __ATOMIC_ACQUIRE); };
+  unsigned long long v = word();
+  for (unsigned n = 1; (unsigned)(v >> 32) != tag; ++n) {
+    if ((n & 1023u) == 0 && std::chrono::steady_clock::now() - start > std::chrono::milliseconds(100)) {
+      HIP_CHECK(hipStreamSynchronize(s));
+      v = word();
+      if ((unsigned)(v >> 32) != tag) throw Error(MPA_ERR_RUNTIME, "max norm: no result from the device");
+      break;
+    }
+    v = word();
+  }
+  const unsigned bits = (unsigned)v;
   float r;
   static_assert(sizeof(r) == sizeof(bits), "float size");
   __builtin_memcpy(&r, &bits, sizeof(r));

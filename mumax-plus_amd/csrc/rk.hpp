@@ -36,11 +36,20 @@ void launch_combine_batch(const CombineJob* jobs, int njobs, hipStream_t s);
 // of the energy minimiser (src/physics/minimizer.cu:59-74).
 void launch_descent(float* m, const float* m0, const float* t, float h, int N, hipStream_t s);
 
-// Reductions write into a small device workspace; results are read back by
-// the caller after a stream synchronisation.
+// Device words of the max norm: the blocks' merged maximum (float bits) and the
+// number of blocks that are done.
+struct NormWords {
+  unsigned max, done;
+};
+
+// Reductions write into a small device workspace; results are read back after
+// a stream synchronisation, the max norm through a word of host memory.
 class Reducer {
  public:
   Reducer();
+  ~Reducer();
+  Reducer(const Reducer&) = delete;
+  Reducer& operator=(const Reducer&) = delete;
   // max over geometry cells of |sum_j c[j] k[j]| (3 components), FP32 norms.
   float max_combo_norm(const Combo& co, int N, const uint8_t* geom, hipStream_t s);
   float max_vec_norm(const float* v, int N, const uint8_t* geom, hipStream_t s);
@@ -57,6 +66,9 @@ class Reducer {
  private:
   DeviceArray<unsigned> maxbits_;
   DeviceArray<double> partials_;
+  DeviceArray<NormWords> words_;
+  unsigned long long* host_ = nullptr;  // pinned: (call number << 32) | float bits
+  unsigned tag_ = 0;
 };
 
 }  // namespace mpa

@@ -2011,12 +2011,12 @@ void TimeSolver::step() {
     double err = 0.0;
     for (auto& sv : vars) {
       Combo co{};
-      co.nk = S;
       for (int j = 0; j < S; ++j) {
-        co.k[j] = (*sv.k)[j].get();
-        co.c[j] = (float)(h * (tb.w1[j] - tb.w2[j]));
+        if (tb.w1[j] == tb.w2[j]) continue;  // adds an exact zero
+        co.k[co.nk] = (*sv.k)[j].get();
+        co.c[co.nk++] = (float)(h * (tb.w1[j] - tb.w2[j]));
       }
-      Timed t(prof, "k_combo_maxnorm", 12.0 * sv.N * S, s);
+      Timed t(prof, "k_combo_maxnorm", 12.0 * sv.N * co.nk, s);
       err = std::max(err, (double)world_->reducer.max_combo_norm(co, sv.N, sv.geom, s));
     }
     const bool success = err < max_error;
