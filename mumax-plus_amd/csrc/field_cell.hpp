@@ -66,6 +66,12 @@ struct FMUniform {
   // one layer (Nz == 1) and no DMI entries along z: the exchange and DMI
   // terms of the two missing (or self-wrapped) z neighbours cancel
   int zflat;
+  // extended path (uniform_extended): per-cell Ms (the coefficients above are
+  // then those of Ms = 1 and scaled per cell) and Ku1, and the Zhang-Li torque
+  // of a uniform current: zl[a] = u_a / (2 c_a), its two factors
+  PS ms, ku;
+  int cells, zhangli;
+  float zl[3], zl1, zl2;
 };
 
 __device__ __forceinline__ float3 gamma_u(const FMUniform& u, int axis, float3 m) { return dmi_gamma(u.D, axis, m); }
@@ -90,10 +96,11 @@ struct NoEpilogue {
 // frozen); zero DMI or anisotropy constants then add exact zeros, and the
 // boundary terms are taken through ghost neighbours (same terms, rounded in
 // another order).
-template <bool FAST = false>
+// EXT: the extended path at cell idx.
+template <bool FAST = false, bool EXT = false>
 __device__ __forceinline__ float3 uniform_result(const FMUniform& u, int mode, float3 mc, const float3 (&mn)[6],
                                                  const bool (&ok)[6], int ndir, bool has_stray, float3 hs,
-                                                 float3 hd) {
+                                                 float3 hd, float ims = 1.f, float ku = 0.f) {
   const bool has_ex = FAST || u.has_ex, has_dmi = FAST || u.has_dmi;
   const bool openbc = !FAST && u.openbc, openbc_dmi = !FAST && u.openbc_dmi;
   const bool uni = FAST || u.uni, cubic = !FAST && u.cubic, demag = FAST || u.demag;
@@ -163,7 +170,7 @@ __device__ __forceinline__ float3 uniform_result(const FMUniform& u, int mode, f
   if (uni) {
     const float3 ua = f3(u.u[0], u.u[1], u.u[2]);
     const float mu = dot3(mc, ua);
-    han = (u.ku1 * mu + u.ku2 * mu * mu * mu) * ua;
+    han = ((EXT ? ku : u.ku1) * mu + u.ku2 * mu * mu * mu) * ua;
   } else if (cubic) {
     const float3 c1 = f3(u.c1[0], u.c1[1], u.c1[2]), c2 = f3(u.c2[0], u.c2[1], u.c2[2]),
                  c3 = f3(u.c3[0], u.c3[1], u.c3[2]);
@@ -173,6 +180,11 @@ __device__ __forceinline__ float3 uniform_result(const FMUniform& u, int mode, f
           u.kc2 * ((s2 * s3) * a1 * c1 + (s1 * s3) * a2 * c2 + (s1 * s2) * a3 * c3) +
           u.kc3 * ((s2 * s2 + s3 * s3) * (s1 * a1) * c1 + (s1 * s1 + s3 * s3) * (s2 * a2) * c2 +
                    (s1 * s1 + s2 * s2) * (s3 * a3) * c3);
+  }
+  if constexpr (EXT) {
+    hex = ims * hex;
+    han = ims * han;
+    hdm = ims * hdm;
   }
   float3 h = hex;
   h = h + han;
@@ -184,7 +196,20 @@ __device__ __forceinline__ float3 uniform_result(const FMUniform& u, int mode, f
   if (!FAST && u.frozen) return f3(0.f, 0.f, 0.f);
   if (FAST || mode == MODE_LLG) {
     const float3 mxh = cross3(mc, h);
-    return u.llg * (mxh + u.alpha * cross3(mc, mxh));
+    const float3 t = u.llg * (mxh + u.alpha * cross3(mc, mxh));
+    if constexpr (EXT) {
+      if (u.zhangli) {
+        // k_ZhangLi, stt.cu:27-102: (u . grad) m by central differences; a
+        // missing neighbour adds nothing
+        float3 g = f3(0.f, 0.f, 0.f);
+#pragma unroll
+        for (int dir = 0; dir < 6; ++dir)
+          if (dir < ndir && ok[dir]) g = g + ((dir & 1) ? u.zl[dir >> 1] : -u.zl[dir >> 1]) * mn[dir];
+        const float3 mxg = cross3(mc, g);
+        return t + (u.zl1 * cross3(mc, mxg) + u.zl2 * mxg);
+      }
+    }
+    return t;
   }
   return -GAMMALL_F * cross3(mc, cross3(mc, h));
 }
@@ -193,7 +218,7 @@ __device__ __forceinline__ float3 uniform_result(const FMUniform& u, int mode, f
 // (the magnet's cell count, or the packed length of a batch); hdem(idx) gives
 // the demag field of the cell (read from memory, or the x-inverse FFT pass's
 // own registers when the field is computed inside that pass).
-template <class HDem, class Epi = NoEpilogue>
+template <bool EXT = false, class HDem, class Epi = NoEpilogue>
 __device__ __forceinline__ void field_uniform_cell(const FMDesc& d, const FMUniform& u, const float* __restrict__ m,
                                                    const HDem& hdem, float* __restrict__ out, int mode, int x, int y,
                                                    int z, int N, const Epi& epi = Epi()) {
@@ -213,7 +238,7 @@ __device__ __forceinline__ void field_uniform_cell(const FMDesc& d, const FMUnif
   const int ndir = u.zflat ? 4 : 6;
   bool ok[6];
   float3 mn[6];
-  if (u.has_ex || u.has_dmi) {
+  if (u.has_ex || u.has_dmi || (EXT && u.zhangli)) {
     int nbi[6];
 #pragma unroll
     for (int dir = 0; dir < 6; ++dir) {
@@ -237,7 +262,16 @@ __device__ __forceinline__ void field_uniform_cell(const FMDesc& d, const FMUnif
   }
   const float3 hs = d.hstray ? load3(d.hstray, idx, d.ncell) : f3(0.f, 0.f, 0.f);
   const float3 hd = u.demag ? hdem(idx) : f3(0.f, 0.f, 0.f);
-  const float3 r = uniform_result(u, mode, mc, mn, ok, ndir, d.hstray != nullptr, hs, hd);
+  float ims = 1.f, ku = u.ku1;
+  if constexpr (EXT) {
+    if (u.cells) {
+      // a cell without moment has no exchange, anisotropy or DMI field
+      const float ms = u.ms.at(idx);
+      ims = ms != 0.f ? 1.f / ms : 0.f;
+      ku = 2.f * u.ku.at(idx);
+    }
+  }
+  const float3 r = uniform_result<false, EXT>(u, mode, mc, mn, ok, ndir, d.hstray != nullptr, hs, hd, ims, ku);
   out[idx] = r.x;
   out[N + idx] = r.y;
   out[2 * N + idx] = r.z;
@@ -399,6 +433,9 @@ __device__ __forceinline__ void field_uniform_b_block_err(const FBInst* __restri
 
 // Every parameter uniform and only the terms the uniform path has.
 bool all_uniform(const FMDesc& d);
+// The uniform path but for per-cell Ms and Ku1, or the Zhang-Li torque of a
+// uniform magnet (the EXT instances).
+bool uniform_extended(const FMDesc& d);
 // Host-side coefficients of the uniform path.
 FMUniform make_uniform(const FMDesc& d);
 

@@ -604,7 +604,8 @@ __global__ void __launch_bounds__(BLOCK) k_torque_pair(FMDesc d0, const float* _
 
 // NK >= 0: also the next stage state, from NK derivatives in memory and the
 // one just computed; NK == -2: none.
-template <int NK>
+// EXT: the extended path.
+template <int NK, bool EXT = false>
 __global__ void __launch_bounds__(BLOCK) k_field_uniform(FMDesc d, FMUniform u, const float* __restrict__ m,
                                                          const float* __restrict__ hdemag, float* __restrict__ out,
                                                          int mode, NextStage next) {
@@ -627,10 +628,10 @@ __global__ void __launch_bounds__(BLOCK) k_field_uniform(FMDesc d, FMUniform u, 
     if (z < d.nz) {
       auto hd = [&](int i) { return load3(hdemag, i, N); };
       if constexpr (NK >= 0)
-        field_uniform_cell(d, u, m, hd, out, mode, x, y, z, N, [&](int idx, float3 mc, float3 r, bool in) {
+        field_uniform_cell<EXT>(d, u, m, hd, out, mode, x, y, z, N, [&](int idx, float3 mc, float3 r, bool in) {
           next.template apply<NK>(idx, mc, r, in);
         });
-      else field_uniform_cell(d, u, m, hd, out, mode, x, y, z, N);
+      else field_uniform_cell<EXT>(d, u, m, hd, out, mode, x, y, z, N);
     }
   }
 }
@@ -638,8 +639,8 @@ __global__ void __launch_bounds__(BLOCK) k_field_uniform(FMDesc d, FMUniform u, 
 // A small magnet's whole evaluation in one launch: the demag field summed
 // directly (demag_direct.hpp), and on the four lanes that hold a strip's
 // fields the field, the torque and (NK >= 0) the next stage state of its
-// cells.  KIND 0: uniform path; 1, 2: per-cell kernel with uniform / any
-// parameters.  Latency-bound: 4 launches of 5 us become one.
+// cells.  KIND 0, 3: uniform path, extended; 1, 2: per-cell kernel with uniform
+// / any parameters.  Latency-bound: 4 launches of 5 us become one.
 template <int KIND, int NK>
 __global__ void __launch_bounds__(1024) k_field_direct(DirectDesc D, FMDesc d, FMUniform u,
                                                        const float* __restrict__ m, float* __restrict__ out, int mode,
@@ -652,13 +653,14 @@ __global__ void __launch_bounds__(1024) k_field_direct(DirectDesc D, FMDesc d, F
   if (!(D.K2 ? direct_sum<false>(D, dlds, red, blockIdx.x, idx, h) : direct_sum<true>(D, dlds, red, blockIdx.x, idx, h)))
     return;
   auto hd = [&](int) { return h; };
-  if constexpr (KIND == 0) {
+  if constexpr (KIND == 0 || KIND == 3) {
     const int x = idx % d.nx, yz = idx / d.nx, y = yz % d.ny, z = yz / d.ny;
     if constexpr (NK >= 0)
-      field_uniform_cell(d, u, m, hd, out, mode, x, y, z, d.ncell, [&](int i, float3 mc, float3 r, bool in) {
-        next.template apply<NK>(i, mc, r, in);
-      });
-    else field_uniform_cell(d, u, m, hd, out, mode, x, y, z, d.ncell);
+      field_uniform_cell<KIND == 3>(d, u, m, hd, out, mode, x, y, z, d.ncell,
+                                    [&](int i, float3 mc, float3 r, bool in) {
+                                      next.template apply<NK>(i, mc, r, in);
+                                    });
+    else field_uniform_cell<KIND == 3>(d, u, m, hd, out, mode, x, y, z, d.ncell);
   } else {
     field_cell<KIND == 1, NK>(d, m, hd, out, mode, idx, &next);
   }
@@ -812,10 +814,30 @@ bool all_uniform(const FMDesc& d) {
          !(d.terms & (TERM_ME | TERM_AFM_NN | TERM_AFM_SITE | TERM_STT | TERM_THERMAL));
 }
 
+// Granular media and current-driven textures otherwise take the per-cell
+// kernel, some 1500 vector instructions and a chain of dependent lookups a
+// cell.  Free boundaries and A not zero: then no rule asks for a neighbour's Ms.
+// 190x150x3 with per-cell Ms and Ku1 14.9-16.8 -> 6.2-7.5 us, 500x100 with
+// the Zhang-Li torque 10.6-11.9 -> 4.9-5.8 us (field with the next stage state).
+bool uniform_extended(const FMDesc& d) {
+  const bool cells = d.msat.p || d.ku1.p, zl = (d.terms & TERM_ZHANGLI) != 0;
+  if (!cells && !zl) return false;
+  FMDesc q = d;
+  q.msat.p = nullptr;
+  q.ku1.p = nullptr;
+  q.terms &= ~TERM_ZHANGLI;
+  if (!all_uniform(q) || d.openbc || d.aex.v == 0.f || !(d.terms & TERM_EXCH) || (d.terms & TERM_CUBIC)) return false;
+  if ((d.terms & TERM_UNI) && d.anisU.x == 0.f && d.anisU.y == 0.f && d.anisU.z == 0.f) return false;
+  if (!d.msat.p && d.msat.v == 0.f) return false;
+  if (!zl) return true;
+  return !cells && !(d.terms & TERM_SLONC) && !d.pol.p && !d.xi.p && !d.jcur.p;
+}
+
 // Host-side coefficients of the uniform path, in double then rounded once.
 FMUniform make_uniform(const FMDesc& d) {
   FMUniform u{};
-  const double ms = d.msat.v, A = d.aex.v;
+  const bool cells = d.msat.p || d.ku1.p;  // scaled per cell by 1 / Ms
+  const double ms = cells ? 1.0 : d.msat.v, A = d.aex.v;
   const double c[3] = {d.cx, d.cy, d.cz};
   const bool msok = ms != 0.0;
   u.has_ex = (d.terms & TERM_EXCH) && msok;
@@ -866,6 +888,20 @@ FMUniform make_uniform(const FMDesc& d) {
   u.alpha = (float)al;
   u.llg = (float)(-1.7595e11 / (1.0 + al * al));
   u.frozen = d.frozen.v != 0.f;
+  u.cells = cells;
+  u.ms = d.msat;
+  u.ku = d.ku1;
+  if (d.terms & TERM_ZHANGLI) {
+    // u = muB pol j / (e Ms (1 + xi^2)); the torque
+    // -1/(1+alpha^2) ((1 + xi alpha) m x (m x g) + (xi - alpha) m x g)
+    const double QEd = 1.60217646e-19, MUBd = 9.274009152e-24, xi = d.xi.v;
+    const double pre = MUBd * d.pol.v / (QEd * ms * (1.0 + xi * xi));
+    const double j[3] = {d.jcur.x, d.jcur.y, d.jcur.z};
+    for (int a = 0; a < 3; ++a) u.zl[a] = (float)(pre * j[a] / (2.0 * c[a]));
+    u.zl1 = (float)(-(1.0 + xi * al) / (1.0 + al * al));
+    u.zl2 = (float)(-(xi - al) / (1.0 + al * al));
+    u.zhangli = 1;
+  }
   return u;
 }
 
@@ -1199,7 +1235,8 @@ std::map<std::array<int, 4>, TileTune>& tile_table() {
 void launch_field_uniform(const FMDesc& d, const float* m, const float* hdemag, float* out, FieldMode mode,
                           const NextStage* next, hipStream_t s) {
   const FMUniform u = make_uniform(d);
-  if (tile_eligible(d)) {
+  const bool ext = uniform_extended(d);
+  if (!ext && tile_eligible(d)) {
     const NextStage ns = next ? *next : NextStage{};
     const bool fast = uniform_fast(d, u, mode);
     auto launch_tile = [&](int zc_req) {
@@ -1271,15 +1308,19 @@ void launch_field_uniform(const FMDesc& d, const float* m, const float* hdemag, 
   dim3 grid((d.nx + bx - 1) / bx, (d.ny + by - 1) / by, (d.nz + MPA_FIELD_ZPER - 1) / MPA_FIELD_ZPER);
   const dim3 blk(bx, by, 1);
   const NextStage ns = next ? *next : NextStage{};
+#define MPA_UNIFORM(K)                                                                      \
+  if (ext) k_field_uniform<K, true><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); \
+  else k_field_uniform<K><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns);
   switch (next ? ns.nk : -2) {
-    case 0: k_field_uniform<0><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); break;
-    case 1: k_field_uniform<1><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); break;
-    case 2: k_field_uniform<2><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); break;
-    case 3: k_field_uniform<3><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); break;
-    case 4: k_field_uniform<4><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); break;
-    case 5: k_field_uniform<5><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); break;
-    default: k_field_uniform<-2><<<grid, blk, 0, s>>>(d, u, m, hdemag, out, (int)mode, ns); break;
+    case 0: MPA_UNIFORM(0) break;
+    case 1: MPA_UNIFORM(1) break;
+    case 2: MPA_UNIFORM(2) break;
+    case 3: MPA_UNIFORM(3) break;
+    case 4: MPA_UNIFORM(4) break;
+    case 5: MPA_UNIFORM(5) break;
+    default: MPA_UNIFORM(-2) break;
   }
+#undef MPA_UNIFORM
   checkLaunch("k_field_uniform");
 }
 }  // namespace
@@ -1314,7 +1355,7 @@ void launch_field_next(const FMDesc& d, const float* m, const float* hdemag, flo
   if (!field_next_fusable(d, mode)) throw Error(MPA_ERR_RUNTIME, "launch_field_next: not a fusable magnet");
   if (next.nk < 0 || next.nk > 5 || !next.out || next.out == m || next.out == out || next.out == next.x0)
     throw Error(MPA_ERR_RUNTIME, "launch_field_next: bad stage combination");
-  if (all_uniform(d)) {
+  if (all_uniform(d) || (uniform_extended(d) && d.nz <= 65535)) {
     launch_field_uniform(d, m, hdemag, out, mode, &next, s);
     return;
   }
@@ -1342,13 +1383,14 @@ void launch_field_direct(const DirectDesc& D, const FMDesc& d, const float* m, f
   if (next && (!field_next_fusable(d, mode) || next->nk < 0 || next->nk > 5 || !next->out || next->out == m ||
                next->out == out || next->out == next->x0))
     throw Error(MPA_ERR_RUNTIME, "launch_field_direct: bad stage combination");
-  const int kind = all_uniform(d) ? 0 : (params_uniform(d) ? 1 : 2);
-  const FMUniform u = kind == 0 ? make_uniform(d) : FMUniform{};
+  const int kind = all_uniform(d) ? 0 : (uniform_extended(d) ? 3 : (params_uniform(d) ? 1 : 2));
+  const FMUniform u = kind == 0 || kind == 3 ? make_uniform(d) : FMUniform{};
   const NextStage ns = next ? *next : NextStage{};
   const DirectLaunch L = direct_launch(D);
 #define MPA_DIRECT(K)                                                                                              \
   switch (kind) {                                                                                                  \
     case 0: k_field_direct<0, K><<<L.blocks, L.threads, L.shm, s>>>(D, d, u, m, out, (int)mode, ns); break;        \
+    case 3: k_field_direct<3, K><<<L.blocks, L.threads, L.shm, s>>>(D, d, u, m, out, (int)mode, ns); break;        \
     case 1: k_field_direct<1, K><<<L.blocks, L.threads, L.shm, s>>>(D, d, u, m, out, (int)mode, ns); break;        \
     default: k_field_direct<2, K><<<L.blocks, L.threads, L.shm, s>>>(D, d, u, m, out, (int)mode, ns); break;       \
   }
@@ -1366,7 +1408,8 @@ void launch_field_direct(const DirectDesc& D, const FMDesc& d, const float* m, f
 }
 
 void launch_field(const FMDesc& d, const float* m, const float* hdemag, float* out, FieldMode mode, hipStream_t s) {
-  if (mode != MODE_EDENS && all_uniform(d) && d.nz <= 65535) {
+  const bool torque = mode == MODE_FIELD || mode == MODE_LLG || mode == MODE_DAMPING;
+  if (mode != MODE_EDENS && d.nz <= 65535 && (all_uniform(d) || (torque && uniform_extended(d)))) {
     launch_field_uniform(d, m, hdemag, out, mode, nullptr, s);
     return;
   }
