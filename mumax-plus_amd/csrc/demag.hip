@@ -339,11 +339,11 @@ __device__ __forceinline__ void xfwd_body(const DD& d, const float* __restrict__
   xfwd_split_store<L2, K>(d, lds, abase, 0, A);
 }
 
-template <int L2, int PLAIN>
-__global__ void __launch_bounds__(XfwdCfg<L2>::THREADS)
+template <int L2, int PLAIN, class K = XfwdCfg<L2>>
+__global__ void __launch_bounds__(K::THREADS)
     k_xfwd(DD d, const float* __restrict__ m, PS msat, const float* __restrict__ m2, PS msat2,
            const uint8_t* __restrict__ geom, float2* __restrict__ A, const float2* __restrict__ tw) {
-  xfwd_body<L2, XfwdCfg<L2>, PLAIN>(d, m, msat, m2, msat2, geom, A, tw, blockIdx.x);
+  xfwd_body<L2, K, PLAIN>(d, m, msat, m2, msat2, geom, A, tw, blockIdx.x);
 }
 
 // x forward with the Runge-Kutta stage combination in front.  The rows of
@@ -848,11 +848,11 @@ __device__ __forceinline__ void xinv_body(const DD& d, const float2* __restrict_
   }
 }
 
-template <int L2>
-__global__ void __launch_bounds__(XinvCfg<L2>::THREADS)
+template <int L2, class K = XinvCfg<L2>>
+__global__ void __launch_bounds__(K::THREADS)
     k_xinv(DD d, const float2* __restrict__ A, const uint8_t* __restrict__ geom, float* __restrict__ h,
            const float2* __restrict__ tw) {
-  xinv_body<L2>(d, A, geom, h, tw, xcd_remap(blockIdx.x, gridDim.x));
+  xinv_body<L2, K>(d, A, geom, h, tw, xcd_remap(blockIdx.x, gridDim.x));
 }
 
 // ---------------------------------------------------------------- y and z of few layers
@@ -1187,17 +1187,39 @@ void make_trig(DeviceArray<double>& ct, DeviceArray<double>& st, int K) {
 
 // ------------------------------------------------ launchers per line length
 
+// Lines of several wavefronts (1024 and 2048 points) have block barriers in
+// their transforms.  With few line pairs the blocks do not fill the chip
+// anyway, and 256 threads wait for fewer wavefronts: 500x100x1 18.5 -> 16.7
+// us for the field, 1000x50x1 19.8 -> 17.7, 300x220x1 (330 pairs) 20.6 -> 19.0.
+// With more pairs the longer runs of 512 threads are faster: 512x512x1 (768
+// pairs) 25.8 against 26.9 us, 800x200x1 (300 pairs of 2048 points) 25.3
+// against 26.0.
+template <int L2>
+bool small_x_blocks(int npairs) {
+  return L2 == 10 ? npairs <= 384 : (L2 == 11 && npairs <= 128);
+}
+
 template <int L2>
 struct RunXfwd {
   static void run(const DD& d, const float* m, PS msat, const float* m2, PS msat2, const uint8_t* geom, float2* A,
                   const float2* tw, hipStream_t s) {
-    using K = XfwdCfg<L2>;
-    const int npairs = (d.nlines + 1) / 2;
-    const dim3 grid = grid_for(npairs, K::PB);
-    if (!geom && !msat.p && !m2) k_xfwd<L2, 1><<<grid, K::THREADS, K::SHM, s>>>(d, m, msat, m2, msat2, geom, A, tw);
+    if constexpr (L2 >= 10) {
+      if (small_x_blocks<L2>((d.nlines + 1) / 2)) {
+        go<XfwdCfgB<L2>>(d, m, msat, m2, msat2, geom, A, tw, s);
+        return;
+      }
+    }
+    go<XfwdCfg<L2>>(d, m, msat, m2, msat2, geom, A, tw, s);
+  }
+  template <class K>
+  static void go(const DD& d, const float* m, PS msat, const float* m2, PS msat2, const uint8_t* geom, float2* A,
+                 const float2* tw, hipStream_t s) {
+    const dim3 grid = grid_for((d.nlines + 1) / 2, K::PB);
+    if (!geom && !msat.p && !m2)
+      k_xfwd<L2, 1, K><<<grid, K::THREADS, K::SHM, s>>>(d, m, msat, m2, msat2, geom, A, tw);
     else if (!geom && !msat.p && !msat2.p)
-      k_xfwd<L2, 2><<<grid, K::THREADS, K::SHM, s>>>(d, m, msat, m2, msat2, geom, A, tw);
-    else k_xfwd<L2, 0><<<grid, K::THREADS, K::SHM, s>>>(d, m, msat, m2, msat2, geom, A, tw);
+      k_xfwd<L2, 2, K><<<grid, K::THREADS, K::SHM, s>>>(d, m, msat, m2, msat2, geom, A, tw);
+    else k_xfwd<L2, 0, K><<<grid, K::THREADS, K::SHM, s>>>(d, m, msat, m2, msat2, geom, A, tw);
     checkLaunch("k_xfwd");
   }
 };
@@ -1282,9 +1304,17 @@ struct YzShm {
 template <int L2>
 struct RunXinv {
   static void run(const DD& d, const float2* A, const uint8_t* geom, float* h, const float2* tw, hipStream_t s) {
-    using K = XinvCfg<L2>;
-    const int npairs = (d.nlines + 1) / 2;
-    k_xinv<L2><<<grid_for(npairs, K::PB), K::THREADS, K::SHM, s>>>(d, A, geom, h, tw);
+    if constexpr (L2 >= 10) {
+      if (small_x_blocks<L2>((d.nlines + 1) / 2)) {
+        go<XinvCfgB<L2>>(d, A, geom, h, tw, s);
+        return;
+      }
+    }
+    go<XinvCfg<L2>>(d, A, geom, h, tw, s);
+  }
+  template <class K>
+  static void go(const DD& d, const float2* A, const uint8_t* geom, float* h, const float2* tw, hipStream_t s) {
+    k_xinv<L2, K><<<grid_for((d.nlines + 1) / 2, K::PB), K::THREADS, K::SHM, s>>>(d, A, geom, h, tw);
     checkLaunch("k_xinv");
   }
 };

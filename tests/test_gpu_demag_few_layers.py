@@ -50,3 +50,10 @@ def test_periodic(pbc):
     mag.magnetization = random_unit(rng, size[::-1]).astype(np.float32)
     want = odemag.demag_fft(mag.magnetization.get().astype(float), 8e5, world.cellsize, None, box, pbc)
     assert np.abs(mag.demag_field() - want).max() <= 6e-7 * np.abs(want).max()
+
+
+# line pairs on either side of the block size rule of the long x lines
+# (1024 points: 384 pairs, 2048 points: 128 pairs)
+@pytest.mark.parametrize("size", [(300, 256, 1), (300, 257, 1), (260, 128, 2), (520, 85, 1), (520, 86, 1)])
+def test_long_x_lines(size):
+    test_field(size)
