@@ -11,6 +11,8 @@
 #include "rk.hpp"
 
 #include <chrono>
+#include <mutex>
+#include <vector>
 
 namespace mpa {
 
@@ -397,21 +399,58 @@ void launch_combine_batch(const CombineJob* jobs, int njobs, hipStream_t s) {
   checkLaunch("k_combine_batch");
 }
 
-Reducer::Reducer() : maxbits_(1), partials_((size_t)3 * SUM_BLOCKS + 3), words_(1) {
-  HIP_CHECK(hipMemset(words_.get(), 0, words_.bytes()));
-  HIP_CHECK(hipStreamSynchronize(nullptr));
-  HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_), sizeof(*host_), hipHostMallocDefault));
-  *host_ = 0;
+namespace {
+// Host words for max norms: one pinned page per process, handed out to the
+// reducers in use (a pinned allocation per world, and its release, would each
+// wait for the whole device).  A reducer past the page's 512 allocates its own.
+constexpr int HOST_WORDS = 512;
+std::mutex host_mu;
+unsigned long long* host_page = nullptr;
+std::vector<int> host_free;
+
+unsigned long long* take_host_word() {
+  std::lock_guard<std::mutex> lk(host_mu);
+  if (!host_page) {
+    HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_page), HOST_WORDS * sizeof(*host_page),
+                            hipHostMallocPortable));
+    for (int i = HOST_WORDS - 1; i >= 0; --i) host_free.push_back(i);
+  }
+  unsigned long long* w = nullptr;
+  if (!host_free.empty()) {
+    w = host_page + host_free.back();
+    host_free.pop_back();
+  } else {
+    HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&w), sizeof(*w), hipHostMallocPortable));
+  }
+  __atomic_store_n(w, 0ull, __ATOMIC_RELEASE);
+  return w;
 }
 
+void give_host_word(unsigned long long* w) {
+  std::lock_guard<std::mutex> lk(host_mu);
+  if (w >= host_page && w < host_page + HOST_WORDS) host_free.push_back((int)(w - host_page));
+  else (void)hipHostFree(w);
+}
+}  // namespace
+
+Reducer::Reducer() : maxbits_(3), partials_((size_t)3 * SUM_BLOCKS + 3) {}
+
 Reducer::~Reducer() {
-  if (host_) (void)hipHostFree(host_);
+  // every norm was waited for, so no launch writes the word any more
+  if (host_) give_host_word(host_);
 }
 
 float Reducer::max_combo_norm(const Combo& co, int N, const uint8_t* geom, hipStream_t s) {
+  NormWords* words = reinterpret_cast<NormWords*>(maxbits_.get() + 1);
+  if (!host_) {
+    host_ = take_host_word();
+    k_zero_u32<<<1, 1, 0, s>>>(&words->max);
+    k_zero_u32<<<1, 1, 0, s>>>(&words->done);
+    checkLaunch("k_zero_u32");
+  }
   const unsigned tag = ++tag_ ? tag_ : ++tag_;  // 0 is the initial content
   const int nb = reduce_blocks(N);
-  auto launch = [&](auto kernel) { kernel<<<nb, BLOCK, 0, s>>>(co, N, geom, words_.get(), host_, tag); };
+  auto launch = [&](auto kernel) { kernel<<<nb, BLOCK, 0, s>>>(co, N, geom, words, host_, tag); };
   switch (co.nk) {
     case 1: launch(k_combo_maxnorm<1>); break;
     case 4: launch(k_combo_maxnorm<4>); break;

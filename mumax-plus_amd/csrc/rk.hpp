@@ -64,10 +64,9 @@ class Reducer {
                double out[3], float* max_dm, hipStream_t s);
 
  private:
-  DeviceArray<unsigned> maxbits_;
+  DeviceArray<unsigned> maxbits_;  // a maximum, then the max norm's NormWords
   DeviceArray<double> partials_;
-  DeviceArray<NormWords> words_;
-  unsigned long long* host_ = nullptr;  // pinned: (call number << 32) | float bits
+  unsigned long long* host_ = nullptr;  // pinned, from the first norm on: (call number << 32) | float bits
   unsigned tag_ = 0;
 };
 

@@ -84,3 +84,32 @@ def test_stepped_torque(size, kind):
     dm, want = mag.magnetization.get() - m0, om.m - m0
     # the step moves m by up to a few percent: its error is that of m (2^-24) over the move
     assert np.abs(dm - want).max() <= 1e-5 * np.abs(want).max() + 1.5e-7
+
+
+def test_two_sublattices():
+    """Ms1 m1 + Ms2 m2 as the source."""
+    size = (33, 25, 1)
+    rng, m = _grid(size)
+    world = mp.World((3e-9, 2e-9, 4e-9))
+    afm = mp.Antiferromagnet(world, mp.Grid(size))
+    afm.sub1.msat, afm.sub2.msat = 6e5, 3e5
+    afm.sub1.magnetization = m
+    afm.sub2.magnetization = random_unit(rng, size[::-1]).astype(np.float32)
+    M = 6e5 * afm.sub1.magnetization.get().astype(float) + 3e5 * afm.sub2.magnetization.get().astype(float)
+    want = odemag.demag_fft(M, 1.0, world.cellsize)
+    assert np.abs(afm.sub1.demag_field() - want).max() <= 4e-7 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("size", [(1, 1024, 3), (3, 1024, 1), (1, 30, 100)])
+def test_most_strips(size):
+    """The widest staging (144 kB of LDS) stays linear and equals its mirror image."""
+    rng, m = _grid(size)
+    world = mp.World((3e-9, 2e-9, 4e-9))
+    mag = mp.Ferromagnet(world, mp.Grid(size))
+    mag.msat = 8e5
+    mag.magnetization = m
+    h = mag.demag_field()
+    flip = mag.magnetization.get()[:, ::-1, ::-1, ::-1].copy()
+    mag.magnetization = flip
+    # a point reflection of the source reflects the field; the sums run in another order
+    assert np.abs(mag.demag_field()[:, ::-1, ::-1, ::-1] - h).max() <= 1e-6 * np.abs(h).max()
