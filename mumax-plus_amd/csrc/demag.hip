@@ -1692,9 +1692,10 @@ DemagPlan::DemagPlan(const DemagGeometry& g) : g_(g) {
 namespace {
 // Grids whose field is summed directly: those where the one launch beats the
 // FFT passes.  Single layers (5 products a pair) up to 4096 cells: 12.3 against
-// 14.0 us there, 5.4 against 12.8 at 960.  More layers (9 products a pair, and
-// five passes on the other side) up to 3584: 12.1 against 19.4 us at 2550.  At
-// 8192 cells the sum takes two to three times the passes.  A batch keeps the
+// 14.0 us there, 5.4 against 12.8 at 960.  More layers (9 products a pair) up
+// to 3584: 7.1 us at 1275 cells and 12.1 at 2550, against 17.9 and 19.4 in five
+// passes or some 13 with the yz pass; in a time step the sum also takes the
+// field launch in.  At 8192 cells the sum takes two to three times the passes.  A batch keeps the
 // passes for every member: it is bound by throughput, where N^2 products lose
 // (256 members of up to 65536 cells: 172 against 91 ms with the members below
 // these limits summed).  Grids of up to 640 cells keep the passes too, so that
