@@ -325,7 +325,7 @@ int mpa_demag_plan_create(const int size[3], const double cellsize[3], const int
 int mpa_demag_plan_destroy(mpa_demag_plan* p);
 /* h = -mu0 N * (Ms m): m, h device arrays of 3*ncells floats; msat_cells device array of ncells
  * floats or NULL (then msat_uniform is used); geometry device array of ncells bytes or NULL;
- * stream: hipStream_t or NULL. */
+ * stream: hipStream_t or NULL.  h may be m (or overlap m or msat_cells). */
 int mpa_demag_plan_exec(mpa_demag_plan* p, const float* m, const float* msat_cells, float msat_uniform,
                         const uint8_t* geometry, float* h, void* stream);
 /* No counterpart in the reference: mpa_demag_plan_exec for callers that cannot allocate device

@@ -1835,9 +1835,22 @@ void DemagPlan::exec_combine(const float* x0, const Combo& co, float* x, PS msat
   run(A_.get(), B_.get(), x, msat, geom, h, s, prof, nullptr, PS{nullptr, 0.f}, &in);
 }
 
+// Whether the 3N field values at h share memory with a source: each block of
+// the direct sum reads the whole source before it writes its own cells, and no
+// order holds between blocks.  The FFT passes have read it all by the time the
+// last of them writes.
+bool DemagPlan::overlaps(const float* h, const float* m, PS msat, const float* m2, PS msat2) const {
+  const uintptr_t h0 = (uintptr_t)h, h1 = h0 + (uintptr_t)3 * N_ * sizeof(float);
+  auto hits = [&](const float* p, int comps) {
+    const uintptr_t p0 = (uintptr_t)p;
+    return p && p0 < h1 && h0 < p0 + (uintptr_t)comps * N_ * sizeof(float);
+  };
+  return hits(m, 3) || hits(msat.p, 1) || hits(m2, 3) || hits(msat2.p, 1);
+}
+
 void DemagPlan::run(float2* A, float2* B, const float* m, PS msat, const uint8_t* geom, float* h, hipStream_t s,
                     Profiler* prof, const float* m2, PS msat2, const StageIn* in) {
-  if (direct_ && !in) {
+  if (direct_ && !in && !overlaps(h, m, msat, m2, msat2)) {
     Timed t(prof, "k_direct", direct_bytes() + (m2 ? 12.0 * N_ : 0.0), s);
     const DirectDesc& D = direct_desc_;
     const DirectLaunch L = direct_launch(D);

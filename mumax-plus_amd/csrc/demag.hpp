@@ -29,7 +29,8 @@ class DemagPlan {
  public:
   explicit DemagPlan(const DemagGeometry& g);
   // h = -mu0 N * (Ms m) on the magnet grid; zero outside the geometry.
-  // m, h: 3*N floats (SoA, x fastest).  geom: N bytes or nullptr.
+  // m, h: 3*N floats (SoA, x fastest); h may be m itself or overlap it.
+  // geom: N bytes or nullptr.
   // prof (optional) times each pass with HIP events.
   // With m2 != nullptr the source is Ms m + Ms2 m2 (the two sublattices of an
   // antiferromagnet, strayfieldfft.cu:206-213).
@@ -57,7 +58,8 @@ class DemagPlan {
   // Whether y, z and the kernel are one pass (two to eight layers).
   bool few() const { return few_; }
   // Whether exec sums the real-space kernel directly (small grids; one
-  // launch, no intermediates), and the description of that sum.
+  // launch, no intermediates; an h that overlaps the source takes the passes),
+  // and the description of that sum.
   bool direct() const { return direct_; }
   const DirectDesc& direct_desc() const { return direct_desc_; }
   double direct_bytes() const;  // algorithmic HBM bytes of the direct sum
@@ -87,6 +89,7 @@ class DemagPlan {
   };
   void run(float2* A, float2* B, const float* m, PS msat, const uint8_t* geom, float* h, hipStream_t s,
            Profiler* prof, const float* m2, PS msat2, const StageIn* in = nullptr);
+  bool overlaps(const float* h, const float* m, PS msat, const float* m2, PS msat2) const;
   size_t a_count() const;
   size_t b_count() const;
   DemagGeometry g_;
