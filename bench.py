@@ -352,14 +352,16 @@ def measure_batch(args, steps):
         dm_default = max(float(np.abs(a.magnetization.get() - b.magnetization.get()).max())
                          for (_, a), (_, b) in zip(members, plain))
         # the same instances through the plain path with the batch's own
-        # kernels (per-cell field kernel, separate stage combination): equal
-        # bit for bit.  The default plain kernels (halo tiles, stage states
-        # in the field launch) round differently in the last bit, and the
-        # random initial states amplify that over 100 steps.
+        # kernels (per-cell field kernel, separate stage combination, demag
+        # by the FFT passes): equal bit for bit.  The default plain kernels
+        # (halo tiles, stage states in the field launch, direct demag sums)
+        # round differently in the last bit, and the random initial states
+        # amplify that over 100 steps.
         matched = [build_batch_member(sp) for sp in specs]
         for w, _ in matched:
             w._impl.set_option("fuse_stages", 0)
             w._impl.set_option("field_zchunk", 0)
+            w._impl.set_option("direct_demag", 0)
             w.timesolver.steps(steps)
         dm = max(float(np.abs(a.magnetization.get() - b.magnetization.get()).max())
                  for (_, a), (_, b) in zip(members, matched))
@@ -404,7 +406,7 @@ def measure_batch(args, steps):
         "sequential": None if wall_seq is None else {
             "value": len(specs) / wall_seq, "unit": "solves/s", "wall_s": wall_seq, "speedup": wall_seq / wall,
             "max_abs_dm_vs_batched": dm, "kernels_for_dm": "plain path with the batch's kernels "
-            "(world options fuse_stages 0, field_zchunk 0)",
+            "(world options fuse_stages 0, field_zchunk 0, direct_demag 0)",
             "max_abs_dm_vs_batched_default_kernels": dm_default},
         "roofline": {"bound": "hbm", "kernel": dom, "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK, "traffic": None,

@@ -368,7 +368,11 @@ int mpa_world_set_profiling(mpa_world* w, int enable);
  * them on the world's stream (the same values).  "split_demag" (default 0): 1 computes the sublattice
  * fields without demag of an antiferromagnet with demag and uniform parameters beside the demag
  * passes and forms its torques after them (the same values bit for bit); 0 computes fields and
- * torques in one launch after the demag passes. */
+ * torques in one launch after the demag passes.  "direct_demag" (default 1): the demag field of a
+ * small magnet is summed directly, in its time steps in the launch that forms the torque; 0 takes
+ * the FFT passes, as "fuse_combine" and a batch do whatever this switch says (the same field to
+ * FP32 rounding; with fuse_stages 0, field_zchunk 0 and direct_demag 0 a magnet's steps equal its
+ * steps in a batch bit for bit). */
 int mpa_world_set_option(mpa_world* w, const char* key, int value);
 int mpa_world_get_option(const mpa_world* w, const char* key, int* value);
 /* The tile-schedule autotuner's record (process-wide; no counterpart in the reference), one line per

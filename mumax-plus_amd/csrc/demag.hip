@@ -1778,9 +1778,9 @@ void DemagPlan::ensure_workspace() {
 }
 
 void DemagPlan::exec(const float* m, PS msat, const uint8_t* geom, float* h, hipStream_t s, Profiler* prof,
-                     const float* m2, PS msat2) {
+                     const float* m2, PS msat2, bool direct) {
   ensure_workspace();
-  run(A_.get(), B_.get(), m, msat, geom, h, s, prof, m2, msat2);
+  run(A_.get(), B_.get(), m, msat, geom, h, s, prof, m2, msat2, direct);
 }
 
 // Scratch of the allocation-free exec: a file-scope device array, one copy per
@@ -1821,7 +1821,7 @@ void DemagPlan::exec_noalloc(const float* m, PS msat, const uint8_t* geom, float
   unsigned char* base = static_cast<unsigned char*>(scratch_address());
   float2* A = reinterpret_cast<float2*>(base);
   float2* B = is2d() ? nullptr : reinterpret_cast<float2*>(base + (a_count() * sizeof(float2) + 255) / 256 * 256);
-  run(A, B, m, msat, geom, h, s, nullptr, nullptr, PS{nullptr, 0.f});
+  run(A, B, m, msat, geom, h, s, nullptr, nullptr, PS{nullptr, 0.f}, true);
 }
 
 void DemagPlan::exec_combine(const float* x0, const Combo& co, float* x, PS msat, const uint8_t* geom, float* h,
@@ -1832,7 +1832,7 @@ void DemagPlan::exec_combine(const float* x0, const Combo& co, float* x, PS msat
     if (co.k[j] == x) throw Error(MPA_ERR_RUNTIME, "demag: stage combination writes a derivative it reads");
   ensure_workspace();
   const StageIn in{x0, &co, x};
-  run(A_.get(), B_.get(), x, msat, geom, h, s, prof, nullptr, PS{nullptr, 0.f}, &in);
+  run(A_.get(), B_.get(), x, msat, geom, h, s, prof, nullptr, PS{nullptr, 0.f}, false, &in);
 }
 
 // Whether the 3N field values at h share memory with a source: each block of
@@ -1849,8 +1849,8 @@ bool DemagPlan::overlaps(const float* h, const float* m, PS msat, const float* m
 }
 
 void DemagPlan::run(float2* A, float2* B, const float* m, PS msat, const uint8_t* geom, float* h, hipStream_t s,
-                    Profiler* prof, const float* m2, PS msat2, const StageIn* in) {
-  if (direct_ && !in && !overlaps(h, m, msat, m2, msat2)) {
+                    Profiler* prof, const float* m2, PS msat2, bool direct, const StageIn* in) {
+  if (direct_ && direct && !overlaps(h, m, msat, m2, msat2)) {
     Timed t(prof, "k_direct", direct_bytes() + (m2 ? 12.0 * N_ : 0.0), s);
     const DirectDesc& D = direct_desc_;
     const DirectLaunch L = direct_launch(D);

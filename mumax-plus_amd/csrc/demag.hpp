@@ -35,9 +35,9 @@ class DemagPlan {
   // With m2 != nullptr the source is Ms m + Ms2 m2 (the two sublattices of an
   // antiferromagnet, strayfieldfft.cu:206-213).
   // The FFT intermediates A and B are the plan's own, allocated on the
-  // first exec.
+  // first exec.  direct: whether a small grid may be summed directly.
   void exec(const float* m, PS msat, const uint8_t* geom, float* h, hipStream_t s, Profiler* prof = nullptr,
-            const float* m2 = nullptr, PS msat2 = PS{nullptr, 0.f});
+            const float* m2 = nullptr, PS msat2 = PS{nullptr, 0.f}, bool direct = true);
   // exec of the Runge-Kutta stage state formed in the first pass:
   // x = normalise(x0 + sum_j co.c[j] co.k[j]), zero outside geom, is written
   // to x (3N floats, not aliasing x0 or any co.k[j]) and its field to h.
@@ -88,7 +88,7 @@ class DemagPlan {
     float* x;
   };
   void run(float2* A, float2* B, const float* m, PS msat, const uint8_t* geom, float* h, hipStream_t s,
-           Profiler* prof, const float* m2, PS msat2, const StageIn* in = nullptr);
+           Profiler* prof, const float* m2, PS msat2, bool direct, const StageIn* in = nullptr);
   bool overlaps(const float* h, const float* m, PS msat, const float* m2, PS msat2) const;
   size_t a_count() const;
   size_t b_count() const;

@@ -806,7 +806,8 @@ void Ferromagnet::ensure_stage_buffers(int S) {
 void Ferromagnet::prepare(unsigned terms, hipStream_t s, Profiler* prof) {
   if (terms & TERM_DEMAG) {
     if (host) host->compute_demag(s, prof);
-    else demag().exec(m.get(), params.at("msat").ps(), geom.get(), hdemag.get(), s, prof);
+    else demag().exec(m.get(), params.at("msat").ps(), geom.get(), hdemag.get(), s, prof, nullptr,
+                        PS{nullptr, 0.f}, world->direct_demag);
   }
   if ((terms & TERM_ME) && !owner()->rigid_strain_applied()) owner()->compute_strain(s);
   if (terms & TERM_EXT) owner()->compute_stray(s, prof);
@@ -941,7 +942,7 @@ void Ferromagnet::eval_rhs(float* out, hipStream_t s, bool prepared, FieldMode m
                            const NextStage* next, bool demag_ready) {
   const unsigned terms = active_terms();
   Profiler* prof = &world->prof;
-  const bool direct = !demag_ready && !host && (terms & TERM_DEMAG) && demag().direct();
+  const bool direct = !demag_ready && direct_rhs(terms);
   if (!prepared) prepare(direct ? terms & ~TERM_DEMAG : terms, s, prof);
   if (direct) {
     // the demag sum reads the magnetisation and writes no field
@@ -962,7 +963,9 @@ void Ferromagnet::eval_rhs(float* out, hipStream_t s, bool prepared, FieldMode m
   launch_field(rhs_desc(terms, noise_dt), m.get(), demag_field(), out, mode, s);
 }
 
-bool Ferromagnet::direct_rhs() { return !host && (active_terms() & TERM_DEMAG) && demag().direct(); }
+bool Ferromagnet::direct_rhs(unsigned terms) {
+  return !host && (terms & TERM_DEMAG) && world->direct_demag && demag().direct();
+}
 
 bool Ferromagnet::next_fusable() {
   if (host || el.enabled) return false;
@@ -1272,7 +1275,7 @@ DemagPlan& Antiferromagnet::demag() {
 // Ms1 m1 + Ms2 m2 (strayfieldfft.cu:206-213), shared by both sublattices.
 void Antiferromagnet::compute_demag(hipStream_t s, Profiler* prof) {
   demag().exec(sub[0]->m.get(), sub[0]->param("msat").ps(), geom.get(), hdemag.get(), s, prof, sub[1]->m.get(),
-               sub[1]->param("msat").ps());
+               sub[1]->param("msat").ps(), world->direct_demag);
 }
 
 int Antiferromagnet::quantity_ncomp(const std::string& q) const {
@@ -1460,8 +1463,9 @@ void World::eval_rhs_all(const std::vector<StateVar>& vars, int stage, hipStream
         if (stage_in)
           fm->demag().exec_combine(stage_in->x0, stage_in->co, fm->m.get(), fm->param("msat").ps(), fm->geom_ptr(),
                                    fm->hdemag.get(), s, &prof);
-        else if ((t & TERM_DEMAG) && !fm->direct_rhs())
-          fm->demag().exec(fm->m.get(), fm->param("msat").ps(), fm->geom_ptr(), fm->hdemag.get(), s, &prof);
+        else if ((t & TERM_DEMAG) && !fm->direct_rhs(t))
+          fm->demag().exec(fm->m.get(), fm->param("msat").ps(), fm->geom_ptr(), fm->hdemag.get(), s, &prof, nullptr,
+                           PS{nullptr, 0.f}, direct_demag);
         fm->eval_rhs(out, s, true, mode, noise_dt, next, stage_in != nullptr);
       }
     } else if (sv.kind == StateVar::DISP) {

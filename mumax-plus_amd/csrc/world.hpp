@@ -259,10 +259,10 @@ class Ferromagnet : public MagnetCore {
   // The right-hand side can also write the next stage state in the same
   // launch (the uniform-parameter LLG path of an independent magnet).
   bool next_fusable();
-  // Whether the right-hand side is one launch with the demag field summed
-  // directly (launch_field_direct): the demag plan's own exec is then not
-  // needed, and hdemag is not written.
-  bool direct_rhs();
+  // Whether a right-hand side with these terms is one launch with the demag
+  // field summed directly (launch_field_direct): the demag plan's own exec is
+  // then not needed, and hdemag is not written.
+  bool direct_rhs(unsigned terms);
   double rhs_bytes(unsigned terms);
   FMDesc rhs_desc(unsigned terms, double noise_dt);
   int eval_quantity(const std::string& q, float* host, hipStream_t s);
@@ -418,6 +418,9 @@ class World {
   // default: at 512 x 512 the field launch fills every compute unit and the
   // demag passes beside it slow down more than the overlap gains.
   bool split_demag = false;
+  // Small magnets' demag fields summed directly (DemagPlan::direct); off: by
+  // the FFT passes, which round as the passes of a batch do.
+  bool direct_demag = true;
 
   // regions: one index per cell, or nullptr (mumaxworld.cpp:57-103)
   Ferromagnet* add_ferromagnet(const int size[3], const int origin[3], const uint8_t* geometry,
