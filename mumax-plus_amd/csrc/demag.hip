@@ -1691,18 +1691,28 @@ DemagPlan::DemagPlan(const DemagGeometry& g) : g_(g) {
 
 namespace {
 // Grids whose field is summed directly: those where the one launch beats the
-// FFT passes.  Single layers (5 products a pair) up to 4096 cells: 12.3 against
-// 14.0 us there, 5.4 against 12.8 at 960.  More layers (9 products a pair) up
-// to 3584: 7.1 us at 1275 cells and 12.1 at 2550, against 17.9 and 19.4 in five
-// passes or some 13 with the yz pass; in a time step the sum also takes the
-// field launch in.  At 8192 cells the sum takes two to three times the passes.  A batch keeps the
-// passes for every member: it is bound by throughput, where N^2 products lose
-// (256 members of up to 65536 cells: 172 against 91 ms with the members below
-// these limits summed).  Grids of up to 640 cells keep the passes too, so that
-// such a magnet's own steps round as its steps in a batch do.
+// FFT passes, alone and in a time step with any parameters.  Its cost is that
+// of strips x units (strips of four x cells, both ny nz ceil(nx / 4)): a row of
+// one cell costs as much as one of four.
+//   Up to 1024 strips, 4096 cells (3584 with layers, 9 products a pair instead
+// of 5): 64x64 11.3 us for the field against 14.3 in passes, 9x340 13.4 against
+// 15.1, 5x16x32 17.4 against 18.9; a Dormand-Prince step 86 against 110 us, 104
+// against 126 and 123 against 144, with per-cell parameters (the general field
+// kernel on four lanes of a wavefront) 161 against 174, 176 against 178 and 194
+// against 199.  Past 1024 strips a block takes eight and loses at once (2x350x3,
+// 1050 strips: a step of 268 against 186 us; 1x30x100: 1230 against 153).
+//   Rows of two to four cells: a lane's kernel entries lie in a line of their
+// own, so up to 768 strips (3x32x24 17.4 against 19.7 us, per-cell steps 196
+// against 205; at 1000 strips 200 against 194).  Rows of one cell have no x
+// transform to save: per-cell steps of 170 against 169 us at 700 strips and 195
+// against 173 at 1000, so none.
+//   A batch keeps the passes for every member: it is bound by throughput, where
+// N^2 products lose (256 members of up to 65536 cells: 172 against 91 ms with
+// the members below these limits summed).  Grids of up to 640 cells keep the
+// passes too, so that their steps round as their steps in a batch do.
 bool direct_rule(int nx, int ny, int nz) {
-  const long long n = (long long)nx * ny * nz;
-  return n > 640 && n <= (nz == 1 ? 4096 : 3584) && (long long)ny * nz * ((nx + 3) / 4) <= 3072;
+  const long long n = (long long)nx * ny * nz, strips = (long long)ny * nz * ((nx + 3) / 4);
+  return nx > 1 && n > 640 && n <= (nz == 1 ? 4096 : 3584) && strips <= (nx <= 4 ? 768 : 1024);
 }
 }  // namespace
 

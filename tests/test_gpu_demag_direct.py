@@ -17,8 +17,8 @@ import mumaxplus as mp
 
 pytestmark = pytest.mark.gpu
 
-# 641 cells and more are summed; the last three lie on the other side of the
-# rule.  No axis is longer than 350 cells: the FP64 tensor's own cancellation
+# 641 cells and more are summed, as far as the rule goes (test_rule): the last
+# three and 2 x 350 x 3 lie on its other side.  No axis is longer than 350 cells: the FP64 tensor's own cancellation
 # (27 terms of r^3 2^-53 / (4 pi) at r cells) is 1e-8 there, but 8e-8 an entry
 # at 700, which the oracle and the device round differently.
 SIZES = [(214, 3, 1), (3, 214, 1), (2, 2, 161), (64, 64, 1), (257, 3, 1), (128, 32, 1), (43, 15, 1), (2, 350, 3),
@@ -100,9 +100,38 @@ def test_two_sublattices():
     assert np.abs(afm.sub1.demag_field() - want).max() <= 4e-7 * np.abs(want).max()
 
 
-@pytest.mark.parametrize("size", [(1, 1024, 3), (3, 1024, 1), (1, 30, 100)])
+# Grids at the edges of the rule (strips of four x cells: 1024, rows of two to
+# four cells 768, rows of one cell none), and whether they are summed.
+RULE = [((64, 64, 1), True), ((13, 256, 1), True), ((5, 256, 4), False), ((5, 16, 32), True), ((5, 171, 3), False),
+        ((4, 256, 3), True), ((4, 193, 4), False), ((2, 32, 24), True), ((2, 350, 3), False), ((1, 30, 100), False),
+        ((1, 55, 55), False), ((1, 350, 2), False), ((641, 1, 1), True), ((32, 20, 1), False), ((65, 64, 1), False)]
+
+
+@pytest.mark.parametrize("size,direct", RULE)
+def test_rule(size, direct):
+    nx, ny, nz = size
+    _, m = _grid(size)
+    world = mp.World((3e-9, 2e-9, 4e-9))
+    mag = mp.Ferromagnet(world, mp.Grid(size))
+    mag.msat, mag.aex, mag.alpha = 8e5, 1.3e-11, 0.1
+    mag.magnetization = m
+    want = odemag.demag_fft(mag.magnetization.get().astype(float), 8e5, world.cellsize)
+    tol = 6e-7 + 3e-15 * max(size) ** 3  # the passes' rounding and the FP64 tensor's own, as for few layers
+    assert np.abs(mag.demag_field() - want).max() <= tol * np.abs(want).max()
+    world.timesolver.adaptive_timestep, world.timesolver.timestep = False, 1e-15
+    world.timesolver.steps(1)
+    impl = world._impl
+    impl.set_profiling(True)
+    impl.profile_reset()
+    world.timesolver.steps(1)
+    names = set(impl.profile_report())
+    impl.set_profiling(False)
+    assert ("k_xfwd" in names) == (not direct), names
+
+
+@pytest.mark.parametrize("size", [(1, 1024, 3), (3, 1024, 1), (1, 30, 100), (13, 256, 1), (1000, 4, 1), (6, 256, 2)])
 def test_most_strips(size):
-    """The widest staging (144 kB of LDS) stays linear and equals its mirror image."""
+    """Long and narrow grids, on both sides of the rule: a field that is not zero and equals its mirror image."""
     rng, m = _grid(size)
     world = mp.World((3e-9, 2e-9, 4e-9))
     mag = mp.Ferromagnet(world, mp.Grid(size))
@@ -111,5 +140,6 @@ def test_most_strips(size):
     h = mag.demag_field()
     flip = mag.magnetization.get()[:, ::-1, ::-1, ::-1].copy()
     mag.magnetization = flip
+    assert np.abs(h).max() > 0.01
     # a point reflection of the source reflects the field; the sums run in another order
     assert np.abs(mag.demag_field()[:, ::-1, ::-1, ::-1] - h).max() <= 1e-6 * np.abs(h).max()
