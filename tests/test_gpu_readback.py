@@ -1,8 +1,11 @@
 """Reads of large fields into numpy arrays, exact: sizes around the threshold of
 the threaded copy (3 MiB) and around its 1 MiB chunks, from one thread and from
-several at once (a second reader takes the plain copy)."""
+several at once (a second reader takes the plain copy), and with a world per
+read (the copy's buffers outlive the worlds that read through them)."""
 
+import gc
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -50,3 +53,34 @@ def test_several_readers():
     assert not bad
     for i, (_, _, want) in enumerate(made):
         assert np.abs(first[i] - want).max() <= 6e-8
+
+
+def _point(n):
+    """One world that reads its state once and goes: seconds of the read and the release, and the state."""
+    world = mp.World((2e-9, 2e-9, 2e-9))
+    mag = mp.Ferromagnet(world, mp.Grid((n, n, 1)))
+    mag.enable_demag = False
+    mag.magnetization = (0.0, 0.6, 0.8)
+    gc.collect()
+    t = time.perf_counter()
+    m = mag.magnetization.get()
+    del mag, world
+    gc.collect()
+    return time.perf_counter() - t, m
+
+
+def test_a_world_per_read():
+    gc.collect()
+    sizes = (500, 512)  # on either side of the threaded copy's threshold
+    for n in sizes:
+        for _ in range(12):  # past the reads that go without the buffers
+            _point(n)
+    took = {n: [] for n in sizes}
+    for _ in range(15):
+        for n in sizes:
+            s, m = _point(n)
+            assert np.array_equal(m[1], np.full((1, n, n), np.float32(0.6)))
+            took[n].append(s)
+    # the larger read has 5 % more bytes; buffers made and freed for each cost
+    # three times the whole
+    assert sorted(took[512])[7] < 1.7 * sorted(took[500])[7]
