@@ -81,6 +81,6 @@ def test_a_world_per_read():
             s, m = _point(n)
             assert np.array_equal(m[1], np.full((1, n, n), np.float32(0.6)))
             took[n].append(s)
-    # the larger read has 5 % more bytes; buffers made and freed for each cost
-    # three times the whole
-    assert sorted(took[512])[7] < 1.7 * sorted(took[500])[7]
+    # 2.9 against 3.1 ms for the read and the release; with buffers made and
+    # freed for each of the larger reads 7.9 against 5.2
+    assert sorted(took[512])[7] < 1.25 * sorted(took[500])[7]
