@@ -400,36 +400,44 @@ void launch_combine_batch(const CombineJob* jobs, int njobs, hipStream_t s) {
 }
 
 namespace {
-// Host words for max norms: one pinned page per process, handed out to the
-// reducers in use (a pinned allocation per world, and its release, would each
-// wait for the whole device).  A reducer past the page's 512 allocates its own.
-constexpr int HOST_WORDS = 512;
+// Host words for max norms, handed out to the reducers in use from pinned
+// pages: a pinned allocation per world, and its release, would each wait for
+// the whole device.  A page more when every word is in use; the pages past the
+// first go when no word is.  The host reads a word while the kernel that wrote
+// it may still run, so the pages are coherent memory.
+constexpr size_t HOST_WORDS = 512;
 std::mutex host_mu;
-unsigned long long* host_page = nullptr;
-std::vector<int> host_free;
+std::vector<unsigned long long*> host_pages, host_free;
+
+void add_host_page(unsigned long long* page) {
+  for (size_t i = HOST_WORDS; i-- > 0;) host_free.push_back(page + i);
+}
 
 unsigned long long* take_host_word() {
   std::lock_guard<std::mutex> lk(host_mu);
-  if (!host_page) {
-    HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_page), HOST_WORDS * sizeof(*host_page),
-                            hipHostMallocPortable));
-    for (int i = HOST_WORDS - 1; i >= 0; --i) host_free.push_back(i);
+  if (host_free.empty()) {
+    host_pages.reserve(host_pages.size() + 1);
+    host_free.reserve((host_pages.size() + 1) * HOST_WORDS);
+    unsigned long long* page = nullptr;
+    HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&page), HOST_WORDS * sizeof(*page),
+                            hipHostMallocPortable | hipHostMallocCoherent));
+    host_pages.push_back(page);
+    add_host_page(page);
   }
-  unsigned long long* w = nullptr;
-  if (!host_free.empty()) {
-    w = host_page + host_free.back();
-    host_free.pop_back();
-  } else {
-    HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&w), sizeof(*w), hipHostMallocPortable));
-  }
+  unsigned long long* w = host_free.back();
+  host_free.pop_back();
   __atomic_store_n(w, 0ull, __ATOMIC_RELEASE);
   return w;
 }
 
 void give_host_word(unsigned long long* w) {
   std::lock_guard<std::mutex> lk(host_mu);
-  if (w >= host_page && w < host_page + HOST_WORDS) host_free.push_back((int)(w - host_page));
-  else (void)hipHostFree(w);
+  host_free.push_back(w);
+  if (host_pages.size() == 1 || host_free.size() < host_pages.size() * HOST_WORDS) return;
+  for (size_t i = 1; i < host_pages.size(); ++i) (void)hipHostFree(host_pages[i]);
+  host_pages.resize(1);
+  host_free.clear();
+  add_host_page(host_pages[0]);
 }
 }  // namespace
 
