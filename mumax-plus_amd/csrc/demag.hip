@@ -1761,6 +1761,8 @@ void DemagPlan::build_kernel(hipStream_t s) {
     k_few_table<<<grid_for((long long)Hx_ * Hy_ * nz), BLOCK, 0, s>>>(t2.get(), Tz_.get(), Hx_, Hy_, nz,
                                                                       -MU0 / ((double)K_[0] * K_[1]));
     checkLaunch("k_few_table");
+    HIP_CHECK(hipStreamSynchronize(s));
+    return;  // no pass of few layers reads the spectrum along z
   }
   DeviceArray<double> t3((size_t)6 * Hz_ * Hy_ * Hx_);
   k_trig_axis<<<grid_for((long long)6 * Hz_ * Hy_ * Hx_), BLOCK, 0, s>>>(t2.get(), t3.get(), 1, nz, Hy_ * Hx_, K_[2],
@@ -2085,15 +2087,14 @@ double DemagPlan::pass_bytes(int i) const {
 double DemagPlan::direct_bytes() const { return (24.0 + (is2d() ? 16.0 : 24.0)) * N_; }
 
 double DemagPlan::algorithmic_bytes() const {
+  if (direct_) return direct_bytes();
   double b = 0.0;
   for (int i = 0; i < npasses(); ++i) b += pass_bytes(i);
   return b;
 }
 
-size_t DemagPlan::device_bytes() const { return A_.bytes() + B_.bytes() + T_.bytes(); }
-
-void DemagPlan::copy_spectrum(float* host) const {
-  HIP_CHECK(hipMemcpy(host, T_.get(), T_.bytes(), hipMemcpyDeviceToHost));
+size_t DemagPlan::device_bytes() const {
+  return A_.bytes() + B_.bytes() + T_.bytes() + Tz_.bytes() + direct_k4_.bytes() + direct_k2_.bytes();
 }
 
 void reference_kernel_size(const DemagGeometry& g, int ksize[3]) {

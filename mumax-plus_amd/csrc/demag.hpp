@@ -71,13 +71,10 @@ class DemagPlan {
   const DemagGeometry& geometry() const { return g_; }
   int K(int a) const { return K_[a]; }
   bool is2d() const { return K_[2] == 1; }
-  // Algorithmic HBM bytes of one exec (see the byte model in the design notes).
+  // Algorithmic HBM bytes of one exec: the direct sum's, or all passes'.
   double algorithmic_bytes() const;
+  // Kernel tables and intermediates held.
   size_t device_bytes() const;
-  // Real kernel spectrum table (Hx x Hy x Hz entries of 6 floats xx, yy, zz,
-  // xy, xz, yz; pre-scaled), for tests.
-  void copy_spectrum(float* host) const;
-  int spectrum_dims(int a) const { return a == 0 ? Hx_ : (a == 1 ? Hy_ : Hz_); }
 
  private:
   friend class DemagBatch;
@@ -98,6 +95,8 @@ class DemagPlan {
   int log2K_[3];
   int Hx_, Hy_, Hz_;
   DeviceArray<float2> A_, B_;
+  // kernel spectrum, Hx x Hy x Hz entries of 6 floats xx, yy, zz, xy, xz, yz
+  // (pre-scaled); few layers have Tz instead
   DeviceArray<float> T_;
   DeviceArray<float2> tw_[3];
   bool few_ = false;

@@ -7,7 +7,7 @@ lengths just outside its rule."""
 import numpy as np
 import pytest
 
-from helpers import random_unit
+from helpers import DeviceBuffer, random_unit
 from oracle import demag as odemag
 
 import mumaxplus as mp
@@ -57,3 +57,29 @@ def test_periodic(pbc):
 @pytest.mark.parametrize("size", [(300, 256, 1), (300, 257, 1), (260, 128, 2), (520, 85, 1), (520, 86, 1)])
 def test_long_x_lines(size):
     test_field(size)
+
+
+def _length(n):
+    k = 8
+    while k < 2 * n - 1:
+        k *= 2
+    return 1 if n == 1 else k
+
+
+@pytest.mark.parametrize("size", [(70, 33, 4), (300, 20, 1), (64, 64, 1), (33, 9, 4), (20, 30, 9)])
+def test_plan_memory(size):
+    """A plan holds the tables that its field needs, and reports them with its intermediates."""
+    nx, ny, nz = size
+    kx, ky, kz = (_length(n) for n in size)
+    hx, hy, hz = kx // 2 + 1, ky // 2 + 1, kz // 2 + 1
+    few = 2 <= nz <= 8
+    # (x, y) spectra of every layer distance, or the whole spectrum: 6 floats an entry
+    tables = 24 * hx * hy * (nz if few else hz)
+    if size in ((64, 64, 1), (33, 9, 4)):  # summed directly: 4 (or 6) floats for dx from -4 nb to 4 nb
+        tables += (16 if nz == 1 else 24) * ny * nz * 8 * ((nx + 3) // 4)
+    plan = mp._cpp.DemagPlan(size, (3e-9, 2e-9, 4e-9))
+    assert plan.info()[2] == tables
+    m, h = DeviceBuffer(12 * nx * ny * nz), DeviceBuffer(12 * nx * ny * nz)
+    plan.exec(m.ptr, h.ptr)
+    a, b = 24 * nz * hx * ny, 0 if nz == 1 or few else 24 * hx * ky * nz
+    assert plan.info()[2] == tables + a + b
