@@ -1684,7 +1684,13 @@ DemagPlan::DemagPlan(const DemagGeometry& g) : g_(g) {
     // the y-lines of a kx in LDS
     size_t shm = 0;
     with_line<YzShm>(log2K_[1], g.n[2], &shm);
-    few_ = shm <= LDS_LIMIT - 1024;
+    // Lines of several wavefronts that take a block of 1024 threads two rounds
+    // want more kx than 17, or the few blocks' serial rounds cost more than the
+    // three launches: 16x512x4 25.6 us for the field against 24.1 in five
+    // passes, 8x1000x2 25.1 against 24.6, 2x355x5 27.0 against 25.6 (with 33 kx
+    // 17x1000x2 26.0 against 27.6, 17x512x4 26.6 against 27.1).
+    const bool rounds = K_[1] >= 1024 && 3 * g.n[2] * K_[1] / 8 > 1024;
+    few_ = shm <= LDS_LIMIT - 1024 && !(rounds && Hx_ <= 17);
   }
   build_kernel(nullptr);
 }

@@ -55,7 +55,8 @@ class DemagPlan {
   size_t workspace_bytes() const;
   // Allocates A and B if the plan does not hold them yet.
   void ensure_workspace();
-  // Whether y, z and the kernel are one pass (two to eight layers).
+  // Whether y, z and the kernel are one pass (two to eight layers, unless
+  // their y lines are long and the grid is narrow along x).
   bool few() const { return few_; }
   // Whether exec sums the real-space kernel directly (small grids; one
   // launch, no intermediates; an h that overlaps the source takes the passes),

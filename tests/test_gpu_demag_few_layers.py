@@ -19,6 +19,9 @@ pytestmark = pytest.mark.gpu
 SIZES = [(150, 30, 2), (90, 20, 3), (70, 20, 4), (60, 15, 5), (50, 15, 6), (40, 17, 7), (40, 17, 8), (40, 15, 9),
          (700, 4, 2), (500, 3, 3), (3, 300, 5), (20, 129, 3), (17, 65, 6), (30, 257, 2), (9, 512, 4), (5, 513, 2),
          (5, 513, 3), (6, 5, 8), (1, 40, 3), (40, 1, 3)]
+# long y lines, which take more than one round, on either side of the width
+# from which they are one pass
+SIZES += [(17, 300, 4), (16, 300, 4), (33, 270, 5), (17, 520, 2), (16, 520, 2), (9, 300, 2), (16, 140, 8)]
 
 
 @pytest.mark.parametrize("size", SIZES)
@@ -66,13 +69,14 @@ def _length(n):
     return 1 if n == 1 else k
 
 
-@pytest.mark.parametrize("size", [(70, 33, 4), (300, 20, 1), (64, 64, 1), (33, 9, 4), (20, 30, 9)])
+@pytest.mark.parametrize("size", [(70, 33, 4), (300, 20, 1), (64, 64, 1), (33, 9, 4), (20, 30, 9), (17, 300, 4),
+                                  (16, 300, 4), (17, 520, 2), (16, 520, 2), (9, 300, 2), (16, 140, 8)])
 def test_plan_memory(size):
     """A plan holds the tables that its field needs, and reports them with its intermediates."""
     nx, ny, nz = size
     kx, ky, kz = (_length(n) for n in size)
     hx, hy, hz = kx // 2 + 1, ky // 2 + 1, kz // 2 + 1
-    few = 2 <= nz <= 8
+    few = 2 <= nz <= 8 and size not in ((16, 300, 4), (16, 520, 2))
     # (x, y) spectra of every layer distance, or the whole spectrum: 6 floats an entry
     tables = 24 * hx * hy * (nz if few else hz)
     if size in ((64, 64, 1), (33, 9, 4)):  # summed directly: 4 (or 6) floats for dx from -4 nb to 4 nb
