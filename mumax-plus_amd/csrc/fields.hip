@@ -1025,7 +1025,10 @@ namespace {
 // not zero on both sides, no mask, no regions that count, no open boundaries,
 // no cubic anisotropy, spin-transfer torque, thermal field, frozen spins or
 // stray field of other magnets, and the magnet within its periodic box.  512 x
-// 512 with the next stage states: 22.6-25.3 -> 12.0-15.0 us.
+// 512 with the next stage states: 22.6-25.3 -> 12.0-15.0 us.  A layer is at
+// least a block, so many layers of a few cells stay on the general kernel (a
+// Dormand-Prince step of 2x2x1000 takes 94 us here and 75 there; 2x2x500
+// 69 and 75, 3x3x1000 65 and 76).
 bool afm_uniform(const FMDesc& a, const FMDesc& b, FieldMode mode) {
   auto one = [](const FMDesc& d) {
     const int n[3] = {d.nx, d.ny, d.nz}, o[3] = {d.ox, d.oy, d.oz}, mg[3] = {d.mgx, d.mgy, d.mgz},
@@ -1036,7 +1039,7 @@ bool afm_uniform(const FMDesc& a, const FMDesc& b, FieldMode mode) {
     if ((d.terms & TERM_UNI) && u[0] == 0.f && u[1] == 0.f && u[2] == 0.f) return false;
     return params_uniform(d) && d.sublattice && d.msat.v != 0.f && d.msat2.v != 0.f && d.aex.v != 0.f && !d.geom &&
            !d.regions && !d.openbc && !d.hstray && !d.noise && d.frozen.v == 0.f && d.latcon.v != 0.f &&
-           !(d.terms & (TERM_CUBIC | TERM_STT | TERM_THERMAL)) && d.nz <= 65535;
+           !(d.terms & (TERM_CUBIC | TERM_STT | TERM_THERMAL)) && (d.nz <= 512 || d.nx * d.ny > 8);
   };
   // terms that are switched per magnet; the pair shares the switches
   const unsigned shared = TERM_EXCH | TERM_DMI | TERM_UNI | TERM_ME | TERM_AFM_NN | TERM_DEMAG;

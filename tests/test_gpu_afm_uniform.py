@@ -18,7 +18,7 @@ CS = (2e-9, 2.5e-9, 3e-9)
 OPEN, FILM = (0, 0, 0), (1, 1, 0)
 CASES = [((65, 5, 1), FILM, True), ((3, 3, 1), FILM, True), ((70, 4, 1), OPEN, True), ((64, 8, 1), (1, 0, 0), True),
          ((5, 1, 1), OPEN, False), ((9, 7, 3), OPEN, True), ((6, 5, 4), (1, 1, 1), True), ((130, 3, 2), FILM, False),
-         ((2, 2, 1), FILM, True)]
+         ((2, 2, 1), FILM, True), ((2, 2, 512), OPEN, False), ((4, 2, 513), OPEN, False), ((3, 3, 513), OPEN, False)]
 
 
 @pytest.mark.parametrize("nn", [0.0, -3e-12])
