@@ -64,10 +64,13 @@ void plain(void* host, const void* dev, size_t bytes, hipStream_t s) {
   HIP_CHECK(hipStreamSynchronize(s));
 }
 
-// Whether a read of this many bytes has the buffers.
-bool ready(size_t bytes) {
+// Whether a read of this many bytes on stream s has the buffers.  Their events
+// belong to one device: a thread that reads with another one current (a host
+// thread starts on device 0, wherever the stream lives) takes the plain copy.
+bool ready(size_t bytes, hipStream_t s) {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return false;
+  hipDevice_t sdev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || hipStreamGetDevice(s, &sdev) != hipSuccess || (int)sdev != dev) return false;
   if (device == dev) return true;
   if (device >= 0) return false;
   plain_bytes += bytes;
@@ -105,7 +108,7 @@ void readback_release() {
 
 void read_back(void* host, const void* dev, size_t bytes, hipStream_t s) {
   std::unique_lock<std::mutex> lk(mu, std::defer_lock);
-  if (bytes < MIN_BYTES || !lk.try_lock() || !ready(bytes)) {
+  if (bytes < MIN_BYTES || !lk.try_lock() || !ready(bytes, s)) {
     plain(host, dev, bytes, s);
     return;
   }
