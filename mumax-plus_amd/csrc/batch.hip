@@ -239,6 +239,7 @@ int Batch::add(Ferromagnet* fm, int mode_flags, double arg) {
   }
   S.active = 1;
   S.accept = 2;  // waiting for its first right-hand side
+  fresh_ = true;
   HIP_CHECK(hipMemcpyAsync(st_.get() + id, &S, sizeof(S), hipMemcpyHostToDevice, stream));
   HIP_CHECK(hipStreamSynchronize(stream));
   dirty_ = true;
@@ -790,15 +791,18 @@ void Batch::advance_passes(long long n) {
 void Batch::advance(long long n) {
   if (n <= 0) return;
   if (broken_) throw Error(MPA_ERR_RUNTIME, "batch: the members' state was lost at a failed grid barrier");
-  std::vector<int> fresh;
-  if (dirty_) {
-    rebuild();
+  if (dirty_) rebuild();
+  // a report since the admission may have rebuilt the tables already: the new
+  // members' first right-hand sides are due all the same
+  if (fresh_) {
+    std::vector<int> fresh;
     std::vector<BatchMember> host(slots_.size());
     HIP_CHECK(hipMemcpy(host.data(), st_.get(), host.size() * sizeof(BatchMember), hipMemcpyDeviceToHost));
     for (size_t i = 0; i < slots_.size(); ++i)
       if (slots_[i].used && host[i].active && host[i].accept == 2) fresh.push_back((int)i);
+    prime(fresh);
+    fresh_ = false;
   }
-  prime(fresh);
   if (nmembers() == 0) return;
   // the per-kernel profile times the per-pass launches
   int mode = prof.enabled ? STEP_PASSES : step_mode;

@@ -154,6 +154,7 @@ class Batch {
   std::unique_ptr<FieldBatch> field0_, field1_;
   double fbytes0_ = 0.0, fbytes1_ = 0.0;  // field launch bytes per group (without the next stage)
   bool dirty_ = true;
+  bool fresh_ = false;  // members were admitted since the last advance
   hipGraph_t graph_ = nullptr;
   hipGraphExec_t exec_ = nullptr;
   // persistent step kernel: phase table, arguments, barrier words

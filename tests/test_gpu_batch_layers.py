@@ -74,3 +74,27 @@ def test_persistent_equals_per_pass(name):
     assert path == "persistent"
     for size, a, b in zip(SHORT[name], got, want):
         assert np.array_equal(a, b), size
+
+
+@pytest.mark.parametrize("mode", ["passes", "persistent"])
+def test_reports_between_admission_and_steps(mode):
+    """Reading the batch's reports after an admission leaves the new member's steps as they are."""
+    sizes = [FLAT, TWO, SEVEN]
+    out = []
+    for ask in (False, True):
+        batch = mp.Batch(8192)
+        batch.step_mode = mode
+        made = [_magnet(s, i) for i, s in enumerate(sizes)]
+        ids = []
+        for _, mag in made:
+            ids.append(batch.add(mag, steps=6))
+            if ask:
+                assert batch.info()["step_bytes"] > 0 and batch.step_path()["persist_grid"] > 0
+            batch.advance(2)
+        while len(batch.finished()) < len(ids):
+            batch.advance(2)
+        for i in ids:
+            batch.remove(i)
+        out.append([mag.magnetization.get() for _, mag in made])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
