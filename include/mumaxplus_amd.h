@@ -350,12 +350,12 @@ int mpa_demag_plan_info(const mpa_demag_plan* p, int fft_size[3], double* algori
  * receives the number of kernel names (at most `cap` are written). */
 int mpa_world_set_profiling(mpa_world* w, int enable);
 /* Stepper switches (no counterpart in the reference).  "fuse_stages" (default 1): a world whose
- * only variable is one magnetisation on the uniform-parameter LLG path, stepped with a
- * first-same-as-last tableau, computes each stage state inside the field launch that produces
- * the last derivative it needs (no separate combination launch); so does a world whose only magnet
- * is one antiferromagnet on the sublattice-pair field kernel (any tableau; its displacement and
- * velocity, with elastodynamics, inside the acceleration launch); 0 runs the separate
- * combination, with the same arithmetic (the same values bit for bit).  "fuse_combine" (default 0): when the only variable is one
+ * only variable is one ferromagnet's magnetisation, without thermal noise, computes each stage state
+ * (and with a tableau that is not first-same-as-last the step's final state) inside the field launch
+ * that produces the last derivative it needs (any parameters and tableau; no separate combination
+ * launch); so does a world whose only magnet is one antiferromagnet on the sublattice-pair field
+ * kernel (its displacement and velocity, with elastodynamics, inside the acceleration launch); 0
+ * runs the separate combination, with the same arithmetic (the same values bit for bit).  "fuse_combine" (default 0): when the only variable is one
  * independent magnetisation with demag, each stage state is formed inside the demag's first FFT
  * pass, which reads the step start and the derivatives instead of the state (no separate
  * combination launch); 0 runs the separate combination.  "field_zchunk" (default 4): z planes per workgroup of the

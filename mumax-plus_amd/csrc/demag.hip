@@ -1946,7 +1946,7 @@ DemagBatch::DemagBatch(const std::vector<Member>& members, long long cs) {
     if (members[j].plan->npasses() == 3) return pass == 0 ? 0 : (pass == 5 ? 2 : 1);
     return pass == 5 ? 4 : pass;
   };
-  // two independent chains: the members with a z transform (group 0) and the
+  // two independent chains: the members of several layers (group 0) and the
   // single layers (group 1)
   for (int group = 0; group < 2; ++group)
   for (int pass : {0, 1, 2, 3, 4, 6, 5}) {

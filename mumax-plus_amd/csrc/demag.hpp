@@ -129,7 +129,7 @@ class DemagBatch {
   // through the events; works under graph capture).
   void exec(const float* X, float* H, hipStream_t s, Profiler* prof, hipStream_t s2 = nullptr,
             hipEvent_t fork = nullptr, hipEvent_t join = nullptr) const;
-  // The passes of one group only (0: members with a z transform, 1: single
+  // The passes of one group only (0: members of several layers, 1: single
   // layers), on stream s.
   void exec_group(const float* X, float* H, int group, hipStream_t s, Profiler* prof) const;
   bool has_group(int group) const;
@@ -139,7 +139,7 @@ class DemagBatch {
   // pass order), for the persistent step kernel.
   struct PassTable {
     int pass;   // 0 xfwd, 1 yfwd, 2 zpass, 3 yinv, 4 ypass2d, 5 xinv, 6 yz
-    int group;  // 0: members with a z transform, 1: single layers
+    int group;  // 0: members of several layers, 1: single layers
     unsigned nblocks;
     size_t shm;
     const void* segs;
@@ -150,7 +150,7 @@ class DemagBatch {
  private:
   struct Launch {
     int pass;   // 0 xfwd, 1 yfwd, 2 zpass, 3 yinv, 4 ypass2d, 5 xinv, 6 yz
-    int group;  // 0: members with a z transform, 1: single layers
+    int group;  // 0: members of several layers, 1: single layers
     bool lean;  // lines of up to 256 points, up to four layers
     size_t shm;
     unsigned nblocks;

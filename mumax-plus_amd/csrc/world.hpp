@@ -257,7 +257,7 @@ class Ferromagnet : public MagnetCore {
   void eval_rhs(float* out, hipStream_t s, bool prepared = false, FieldMode mode = MODE_LLG, double noise_dt = 0.0,
                 const NextStage* next = nullptr, bool demag_ready = false);
   // The right-hand side can also write the next stage state in the same
-  // launch (the uniform-parameter LLG path of an independent magnet).
+  // launch (an independent magnet without elastodynamics or thermal noise).
   bool next_fusable();
   // Whether a right-hand side with these terms is one launch with the demag
   // field summed directly (launch_field_direct): the demag plan's own exec is
@@ -357,7 +357,7 @@ class TimeSolver {
   // stage combinations inside the field launch where possible (one read of
   // the last derivative less per stage): 2.30 against 2.32 ms per step at
   // 256x256x64 on MI355X; for a lone antiferromagnet inside its
-  // sublattice-field and acceleration launches: 0.431 against 0.4545 ms per
+  // sublattice-field and acceleration launches: 0.318 against 0.335 ms per
   // step at 512x512 with elastodynamics
   bool fuse_stages = true;
   // the stage combination of a lone magnetisation with demag inside the
